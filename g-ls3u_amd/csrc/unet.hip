@@ -180,17 +180,14 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
   __bf16* ge_top = nullptr;
   for (int l = 0; l <= Lv - 2; ++l) {
     const int Hl = H >> l, Wl = W >> l;
-    const long Pl = (long)n * Hl * Wl;
     const int Cl = h->C(l), Cn = h->C(l + 1);
     Layer& la = h->dec(l, 0);
     Layer& lb = h->dec(l, 1);
     const __bf16* low = (l + 1 <= Lv - 2) ? a.d[l + 1] : a.e[Lv - 1];
-    UTRY(unet_conv3_dw(a.gd[l], Cl, a.da[l], Cl, nullptr, 0, lb.gw, n, Hl, Wl, s));
-    UTRY(unet_bias_grad(a.gd[l], lb.gb, Pl, Cl, s));
+    UTRY(unet_conv3_dw(a.gd[l], Cl, a.da[l], Cl, nullptr, 0, lb.gw, lb.gb, n, Hl, Wl, s));
     UTRY(unet_conv3(a.gd[l], Cl, nullptr, 0, lb.wt, nullptr, a.da[l], a.gda[l], n, Hl, Wl, Cl, 1,
                     s));
-    UTRY(unet_conv3_dw(a.gda[l], Cl, a.e[l], Cl, low, Cn, la.gw, n, Hl, Wl, s));
-    UTRY(unet_bias_grad(a.gda[l], la.gb, Pl, Cl, s));
+    UTRY(unet_conv3_dw(a.gda[l], Cl, a.e[l], Cl, low, Cn, la.gw, la.gb, n, Hl, Wl, s));
     UTRY(unet_conv3(a.gda[l], Cl, nullptr, 0, la.wt, nullptr, nullptr, a.gcat[l], n, Hl, Wl,
                     Cl + Cn, 1, s));
     __bf16* gl = (l + 1 <= Lv - 2) ? a.gd[l + 1] : a.ge[Lv - 1];
@@ -201,12 +198,10 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
   (void)ge_top;
   for (int l = Lv - 1; l >= 0; --l) {
     const int Hl = H >> l, Wl = W >> l;
-    const long Pl = (long)n * Hl * Wl;
     const int Cl = h->C(l);
     Layer& la = h->enc(l, 0);
     Layer& lb = h->enc(l, 1);
-    UTRY(unet_conv3_dw(a.ge[l], Cl, a.ea[l], Cl, nullptr, 0, lb.gw, n, Hl, Wl, s));
-    UTRY(unet_bias_grad(a.ge[l], lb.gb, Pl, Cl, s));
+    UTRY(unet_conv3_dw(a.ge[l], Cl, a.ea[l], Cl, nullptr, 0, lb.gw, lb.gb, n, Hl, Wl, s));
     UTRY(unet_conv3(a.ge[l], Cl, nullptr, 0, lb.wt, nullptr, a.ea[l], a.gea[l], n, Hl, Wl, Cl, 1,
                     s));
     if (l == 0) {
@@ -214,8 +209,7 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
       break;
     }
     const int Cp = h->C(l - 1);
-    UTRY(unet_conv3_dw(a.gea[l], Cl, a.p[l - 1], Cp, nullptr, 0, la.gw, n, Hl, Wl, s));
-    UTRY(unet_bias_grad(a.gea[l], la.gb, Pl, Cl, s));
+    UTRY(unet_conv3_dw(a.gea[l], Cl, a.p[l - 1], Cp, nullptr, 0, la.gw, la.gb, n, Hl, Wl, s));
     UTRY(unet_conv3(a.gea[l], Cl, nullptr, 0, la.wt, nullptr, nullptr, a.gp[l - 1], n, Hl, Wl, Cp,
                     1, s));
     UTRY(unet_pool_bwd(a.e[l - 1], a.gp[l - 1], a.gcat[l - 1], Cp + Cl, a.ge[l - 1], n, H >> (l - 1),

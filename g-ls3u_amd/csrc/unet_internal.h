@@ -13,9 +13,10 @@ namespace glsu {
 hipError_t unet_conv3(const __bf16* X1, int C1, const __bf16* X2, int C2, const __bf16* Wt,
                       const float* bias, const __bf16* mask, __bf16* Y, int n, int H, int W,
                       int Cout, int mode, hipStream_t s, __bf16* pool = nullptr);
-// dW [Cout][9][Cin] += weight gradient (FP32, atomically accumulated)
+// dW [Cout][9][Cin] += weight gradient, db [Cout] += bias gradient (FP32,
+// atomically accumulated)
 hipError_t unet_conv3_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
-                         int C2, float* dW, int n, int H, int W, hipStream_t s);
+                         int C2, float* dW, float* db, int n, int H, int W, hipStream_t s);
 hipError_t unet_conv3_in(const float2* x, const float* w, const float* b, __bf16* Y, int n,
                          int H, int W, int C0, hipStream_t s);
 hipError_t unet_conv3_in_dw(const float2* x, const __bf16* dY, float* dW, float* db, int n,
@@ -30,7 +31,6 @@ hipError_t unet_pool_bwd(const __bf16* e, const __bf16* gp, const __bf16* gskip,
                          __bf16* ge, int n, int H, int W, int C, hipStream_t s);
 hipError_t unet_up_bwd(const __bf16* gcat, int C1, const __bf16* a, __bf16* ga, int n, int H2,
                        int W2, int C, hipStream_t s);
-hipError_t unet_bias_grad(const __bf16* g, float* db, long P, int C, hipStream_t s);
 hipError_t unet_adam(float* w, const float* g, float* m, float* v, long count, float lr,
                      float b1, float b2, float eps, int step, hipStream_t s);
 hipError_t unet_weights_bf16(const float* w, __bf16* wf, __bf16* wt, int Cout, int Cin,

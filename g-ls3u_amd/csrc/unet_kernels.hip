@@ -758,76 +758,238 @@ __global__ __launch_bounds__(512, 1) void conv3_res64_kernel(
 }
 
 // ------------------------------------------------------------------------
-// Weight gradient of a 3x3 convolution: dW[co][t][ci] += sum_p dY[p][co] *
-// X[p + off_t][ci], one tap per workgroup (blockIdx.z), a 64 x 64 (co, ci)
-// tile (blockIdx.y) and a range of pixels (blockIdx.x, split K; partial sums
-// are added to the FP32 gradient atomically).  32-pixel chunks of dY and of
-// the shifted input are staged transposed in LDS ([channel][pixel]) so that
-// both MFMA operands are 16-byte LDS reads of 8 consecutive pixels.
-constexpr int kDwPix = 32, kDwPad = 40;
+// Weight and bias gradient of a 3x3 convolution: dW[co][t][ci] += sum_p
+// dY[p][co] * X[p + off_t][ci], db[co] += sum_p dY[p][co], on BF16 MFMA with
+// the pixels as the contraction axis.
+//
+// A wave owns a 32 x 32 (co, ci) block of ALL nine taps (144 accumulator
+// registers) over a strip 32 pixels wide, and marches down the strip's rows:
+// per input row it reads one new dY row (the two before stay in registers)
+// and the input row once per tap column dx, and issues all 36 MFMAs of the
+// nine taps on them, so dY and X are read once per (co, ci) tile instead of
+// once per tap.  NHWC rows are staged in LDS as they lie in memory; the MFMA
+// operands (8 pixels of one channel per lane) come out of LDS through the
+// transposing read ds_read_b64_tr_b16, which takes a 4-pixel x 16-channel
+// block per 16 lanes, so no transposed copy is written.  The order of the 32
+// pixels along K is the same permutation for both operands.
+// LDS pixels are 32 ch + 16 elements apart: the four pixels of a 16-lane read
+// then lie in four different 32-byte bank groups.
+//
+// Workgroup: MB x NB blocks of 32 x 32 channels times S strips (one wave
+// each); R rows are staged at a time, double-buffered, the next rows' global
+// loads in flight during the MFMAs.  The rows of all images are one sequence
+// with a zero row after each image (img * (H + 1) + y), cut into chunks, one
+// per workgroup, so the launch fills the chip whatever n, H and W are; strips
+// are summed through LDS and chunks by FP32 atomics.
+// Bound at full resolution (32 channels) by memory, above it by LDS reads
+// (16 transposing reads per 36 MFMAs) and the MFMAs.
+constexpr int kGrStrip = 32;
 
-__global__ __launch_bounds__(256) void conv3_dw_kernel(
+__device__ __forceinline__ bf16x8 lds_tr8(const __bf16* p0, const __bf16* p1) {
+  typedef short v4s __attribute__((ext_vector_type(4)));
+  typedef __attribute__((address_space(3))) v4s* lp;
+  union {
+    v4s h[2];
+    bf16x8 v;
+  } u;
+  u.h[0] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)p0);
+  u.h[1] = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lp)p1);
+  return u.v;
+}
+
+template <int MB, int NB, int S, int R>
+struct GradConv {
+  static constexpr int Threads = 64 * MB * NB * S;
+  static constexpr int XP = 32 * NB + 16, YP = 32 * MB + 16;  // LDS pixel pitch (elements)
+  static constexpr int XW = kGrStrip * S + 2, YW = kGrStrip * S;
+  static constexpr int XRow = XW * XP, YRow = YW * YP;        // elements
+  static constexpr int Stage = R * (XRow + YRow);
+  static constexpr int XSlots = XW * NB * 4, YSlots = YW * MB * 4;  // 16-byte slots of a row
+  static constexpr int XLd = (XSlots + Threads - 1) / Threads;
+  static constexpr int YLd = (YSlots + Threads - 1) / Threads;
+  // strip sums go through LDS, one tap at a time, after the main loop
+  static_assert(S == 1 || MB * NB * (S - 1) * 4096 <= 2 * Stage * 2, "strip sums fit the stages");
+};
+
+template <int MB, int NB, int S, int R>
+__global__ __launch_bounds__(64 * MB * NB * S) void conv3_dw_kernel(
     const __bf16* __restrict__ dY, int Cout, const __bf16* __restrict__ X1, int C1,
-    const __bf16* __restrict__ X2, int C2, float* __restrict__ dW, int n, int H, int W,
-    int pix_per_block) {
-  __shared__ __attribute__((aligned(16))) __bf16 sA[64 * kDwPad];  // [co][pixel]
-  __shared__ __attribute__((aligned(16))) __bf16 sB[64 * kDwPad];  // [ci][pixel]
+    const __bf16* __restrict__ X2, int C2, float* __restrict__ dW, float* __restrict__ db, int n,
+    int H, int W, int rows_per_wg) {
+  using G = GradConv<MB, NB, S, R>;
+  __shared__ __attribute__((aligned(16))) __bf16 sm[2][G::Stage];
   const int Cin = C1 + C2;
-  const int t = blockIdx.z, dy = t / 3 - 1, dx = t % 3 - 1;
-  const int nci = (Cin + 63) / 64;
-  const int co0 = (blockIdx.y / nci) * 64, ci0 = (blockIdx.y % nci) * 64;
-  const long P = (long)n * H * W;
-  const long p0 = (long)blockIdx.x * pix_per_block;
-  const long p1 = std::min(P, p0 + pix_per_block);
-  const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-  const int lr = lane % 16, lk = lane / 16;
-  const int wm = wave / 2, wn = wave % 2;  // wave tile: co [32 wm, +32), ci [32 wn, +32)
-  floatx4 acc[2][2];
+  const int ncx = Cin / (32 * NB);
+  const int co0 = (blockIdx.y / ncx) * 32 * MB, ci0 = (blockIdx.y % ncx) * 32 * NB;
+  const int x0 = blockIdx.z * kGrStrip * S;
+  const int V = n * (H + 1);  // rows of all images, each followed by a zero row
+  const int v0 = blockIdx.x * rows_per_wg, v1 = min(V, v0 + rows_per_wg);
+  const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
+  const int s = wave / (MB * NB), wm = (wave / NB) % MB, wn = wave % NB;
+  // the source of this workgroup's input channels (never straddles the two)
+  const bool low = ci0 >= C1;
+  const __bf16* __restrict__ X = low ? X2 + (ci0 - C1) : X1 + ci0;
+  const int Cx = low ? C2 : C1, sh = low ? 1 : 0, Hx = H >> sh, Wx = W >> sh;
+
+  // this thread's slots of a row: element offset in the source row, LDS
+  // offset, and whether the pixel is in the image
+  int xo[G::XLd], yo[G::YLd];
+  unsigned xin = 0, yin = 0;
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
-#pragma unroll
-    for (int j = 0; j < 2; ++j) acc[i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-  // staging role of this thread: pixel sp of the chunk, 8-channel group sg
-  const int sp = threadIdx.x / 8, sg = threadIdx.x % 8;
-  for (long pc = p0; pc < p1; pc += kDwPix) {
-    const long p = pc + sp;
-    bf16x8 va = zero8(), vb = zero8();
-    if (p < p1) {
-      const int x = (int)(p % W), y = (int)((p / W) % H), img = (int)(p / ((long)W * H));
-      const int co = co0 + sg * 8, ci = ci0 + sg * 8;
-      if (co < Cout) va = *(const bf16x8*)(dY + (size_t)p * Cout + co);
-      if (ci < Cin) vb = load8(X1, C1, X2, C2, img, y + dy, x + dx, H, W, ci);
-    }
-    __syncthreads();  // previous chunk consumed
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      sA[(sg * 8 + i) * kDwPad + sp] = va[i];
-      sB[(sg * 8 + i) * kDwPad + sp] = vb[i];
-    }
-    __syncthreads();
-    bf16x8 a[2], b[2];
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      a[i] = *(const bf16x8*)(sA + (wm * 32 + i * 16 + lr) * kDwPad + lk * 8);
-      b[i] = *(const bf16x8*)(sB + (wn * 32 + i * 16 + lr) * kDwPad + lk * 8);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-      for (int j = 0; j < 2; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b[j], acc[i][j], 0, 0, 0);
+  for (int k = 0; k < G::XLd; ++k) {
+    const int i = tid + G::Threads * k, px = i / (NB * 4), g = i % (NB * 4), x = x0 - 1 + px;
+    xin |= (x >= 0 && x < W ? 1u : 0u) << k;
+    xo[k] = (min(max(x, 0), W - 1) >> sh) * Cx + g * 8;
   }
-  // acc[i][j][r]: co = co0 + 32 wm + 16 i + 4 lk + r, ci = ci0 + 32 wn + 16 j + lr
 #pragma unroll
-  for (int i = 0; i < 2; ++i)
+  for (int k = 0; k < G::YLd; ++k) {
+    const int i = tid + G::Threads * k, px = i / (MB * 4), g = i % (MB * 4), x = x0 + px;
+    yin |= (x < W ? 1u : 0u) << k;
+    yo[k] = min(x, W - 1) * Cout + co0 + g * 8;
+  }
+  bf16x8 lx[R][G::XLd], ly[R][G::YLd];
+  // input rows v .. v + R - 1 and the dY rows one below them
+  auto load = [&](int v) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const int vi = v + r, vo = vi + 1;
+      const int im = max(vi, 0) / (H + 1), y = vi - im * (H + 1);
+      const bool live = vi >= 0 && vi < V && y < H;  // uniform
+      const __bf16* b = X + ((size_t)min(im, n - 1) * Hx + (min(max(y, 0), H - 1) >> sh)) * Wx * Cx;
+#pragma unroll
+      for (int k = 0; k < G::XLd; ++k) {
+        const bf16x8 t = *(const bf16x8*)(b + xo[k]);
+        lx[r][k] = live && ((xin >> k) & 1) ? t : zero8();
+      }
+      const int om = vo / (H + 1), q = vo - om * (H + 1);
+      const bool olive = vo < v1 && q < H;  // vo >= v0 always
+      const __bf16* d = dY + ((size_t)min(om, n - 1) * H + min(q, H - 1)) * W * Cout;
+#pragma unroll
+      for (int k = 0; k < G::YLd; ++k) {
+        const bf16x8 t = *(const bf16x8*)(d + yo[k]);
+        ly[r][k] = olive && ((yin >> k) & 1) ? t : zero8();
+      }
+    }
+  };
+  auto store = [&](__bf16* buf) {
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      __bf16* bx = buf + r * (G::XRow + G::YRow);
+      __bf16* by = bx + G::XRow;
+#pragma unroll
+      for (int k = 0; k < G::XLd; ++k) {
+        const int i = tid + G::Threads * k;
+        if (i < G::XSlots) *(bf16x8*)(bx + (i / (NB * 4)) * G::XP + (i % (NB * 4)) * 8) = lx[r][k];
+      }
+#pragma unroll
+      for (int k = 0; k < G::YLd; ++k) {
+        const int i = tid + G::Threads * k;
+        if (i < G::YSlots) *(bf16x8*)(by + (i / (MB * 4)) * G::YP + (i % (MB * 4)) * 8) = ly[r][k];
+      }
+    }
+  };
+
+  floatx4 acc[9][2][2], accb[2];
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    accb[i] = floatx4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 2; ++j)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) {
-        const int co = co0 + 32 * wm + 16 * i + 4 * lk + r;
-        const int ci = ci0 + 32 * wn + 16 * j + lr;
-        if (co < Cout && ci < Cin) atomicAdd(dW + ((size_t)co * 9 + t) * Cin + ci, acc[i][j][r]);
+      for (int t = 0; t < 9; ++t) acc[t][i][j] = floatx4{0.f, 0.f, 0.f, 0.f};
+  }
+  bf16x8 a0[2], a1[2], a2[2], ones;  // dY rows vi - 1, vi, vi + 1
+#pragma unroll
+  for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.f;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) a1[i] = a2[i] = zero8();
+  const bool bias = ci0 == 0 && wn == 0;
+  // transposing read: lane l of a 16-lane group addresses pixel l / 4, channels
+  // 4 (l % 4) .. + 3, and receives channel l of the four pixels; group lk reads
+  // pixels 4 lk + (0..3) and, for the second half of K, 16 + 4 lk + (0..3)
+  const int lpx = 4 * (lane / 16) + (lane % 16) / 4, lch = (lane % 4) * 4;
+  const int xbase = (kGrStrip * s + lpx) * G::XP + wn * 32 + lch;
+  const int ybase = (kGrStrip * s + lpx) * G::YP + wm * 32 + lch;
+
+  load(v0 - 1);
+  store(sm[0]);
+  __syncthreads();
+  int cur = 0;
+  for (int v = v0 - 1; v <= v1; v += R, cur ^= 1) {
+    const bool more = v + R <= v1;
+    if (more) load(v + R);
+#pragma unroll
+    for (int r = 0; r < R; ++r) {
+      const __bf16* bx = sm[cur] + r * (G::XRow + G::YRow) + xbase;
+      const __bf16* by = sm[cur] + r * (G::XRow + G::YRow) + G::XRow + ybase;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        a0[i] = a1[i];
+        a1[i] = a2[i];
+        a2[i] = lds_tr8(by + i * 16, by + i * 16 + 16 * G::YP);
       }
+      if (bias) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+          accb[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[i], ones, accb[i], 0, 0, 0);
+      }
+#pragma unroll
+      for (int dx = 0; dx < 3; ++dx) {
+        bf16x8 b[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+          b[j] = lds_tr8(bx + dx * G::XP + j * 16, bx + (dx + 16) * G::XP + j * 16);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < 2; ++j) {
+            // output row one below, at and above the input row: tap rows 0, 1, 2
+            acc[dx][i][j] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[i], b[j], acc[dx][i][j], 0, 0, 0);
+            acc[3 + dx][i][j] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[i], b[j], acc[3 + dx][i][j], 0, 0, 0);
+            acc[6 + dx][i][j] =
+                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[i], b[j], acc[6 + dx][i][j], 0, 0, 0);
+          }
+      }
+    }
+    if (more) store(sm[cur ^ 1]);
+    __syncthreads();
+  }
+  // acc[t][i][j][r]: co = co0 + 32 wm + 16 i + 4 lk + r, ci = ci0 + 32 wn + 16 j + lr
+  const int lr = lane % 16, lk = lane / 16;
+  float* red = (float*)&sm[0][0];
+  const int blk = wave % (MB * NB);
+#pragma unroll
+  for (int t = 0; t < 9; ++t) {
+    if constexpr (S > 1) {
+      if (s > 0) {
+        float* o = red + ((s - 1) * MB * NB + blk) * 1024 + lane;
+#pragma unroll
+        for (int k = 0; k < 16; ++k) o[64 * k] = acc[t][k / 8][(k / 4) % 2][k % 4];
+      }
+      __syncthreads();
+    }
+    if (s == 0) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int i = k / 8, j = (k / 4) % 2, r = k % 4;
+        float v = acc[t][i][j][r];
+#pragma unroll
+        for (int q = 0; q < S - 1; ++q) v += red[(q * MB * NB + blk) * 1024 + 64 * k + lane];
+        const int co = co0 + 32 * wm + 16 * i + 4 * lk + r, ci = ci0 + 32 * wn + 16 * j + lr;
+        atomicAdd(dW + ((size_t)co * 9 + t) * Cin + ci, v);
+      }
+    }
+    if constexpr (S > 1) __syncthreads();
+  }
+  if (bias && lr == 0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        atomicAdd(db + co0 + 32 * wm + 16 * i + 4 * lk + r, accb[i][r]);
+  }
 }
 
 // ------------------------------------------------------------------------
@@ -1073,18 +1235,6 @@ __global__ __launch_bounds__(256) void up_bwd_kernel(const __bf16* __restrict__ 
   ga[q * C + c] = (__bf16)(((float)a[q * C + c] > 0.f) ? s : 0.f);
 }
 
-// db[c] += sum_p g[p][c]
-__global__ __launch_bounds__(256) void bias_grad_kernel(const __bf16* __restrict__ g,
-                                                        float* __restrict__ db, long P, int C,
-                                                        int pix_per_block) {
-  const int c = threadIdx.x;
-  if (c >= C) return;
-  const long p0 = (long)blockIdx.x * pix_per_block, p1 = std::min(P, p0 + pix_per_block);
-  float s = 0.f;
-  for (long p = p0; p < p1; ++p) s += (float)g[(size_t)p * C + c];
-  atomicAdd(db + c, s);
-}
-
 // Adam on FP32 master weights; refreshes the BF16 copies: Wf [Cout][9][Cin]
 // and, for 3x3 layers, the flipped transpose Wt [Cin][9][Cout].
 __global__ __launch_bounds__(256) void adam_kernel(float* __restrict__ w,
@@ -1201,16 +1351,40 @@ hipError_t unet_conv3(const __bf16* X1, int C1, const __bf16* X2, int C2, const 
   return unet_maxpool2(Y, pool, n, H, W, Cout, s);
 }
 
-hipError_t unet_conv3_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
-                         int C2, float* dW, int n, int H, int W, hipStream_t s) {
-  if ((C1 % 32) || (C2 % 32) || (Cout % 32)) return hipErrorInvalidValue;
-  const long P = (long)n * H * W;
-  const int ppb = 4096;
-  const int tilesc = ((Cout + 63) / 64) * ((C1 + C2 + 63) / 64);
-  dim3 grid((unsigned)((P + ppb - 1) / ppb), tilesc, 9);
-  hipLaunchKernelGGL(conv3_dw_kernel, grid, dim3(256), 0, s, dY, Cout, X1, C1, X2, C2, dW, n, H,
-                     W, ppb);
+template <int MB, int NB, int S, int R>
+static hipError_t launch_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
+                            int C2, float* dW, float* db, int n, int H, int W, int wgs,
+                            hipStream_t s) {
+  using G = GradConv<MB, NB, S, R>;
+  const int tiles = (Cout / (32 * MB)) * ((C1 + C2) / (32 * NB));
+  const int strips = (W + kGrStrip * S - 1) / (kGrStrip * S);
+  // chunks of rows: as many as fill the chip once, but at least six rows each
+  // (every chunk reads two input rows more than it owns)
+  const int V = n * (H + 1);
+  const int chunks = std::max(1, std::min(wgs / std::max(1, tiles * strips), V / 6));
+  const int rows = (V + chunks - 1) / chunks;
+  hipLaunchKernelGGL((conv3_dw_kernel<MB, NB, S, R>), dim3((V + rows - 1) / rows, tiles, strips),
+                     dim3(G::Threads), 0, s, dY, Cout, X1, C1, X2, C2, dW, db, n, H, W, rows);
   return hipGetLastError();
+}
+
+hipError_t unet_conv3_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
+                         int C2, float* dW, float* db, int n, int H, int W, hipStream_t s) {
+  if ((C1 % 32) || (C2 % 32) || (Cout % 32) || (C2 && ((H | W) & 1))) return hipErrorInvalidValue;
+  static int cus = 0;
+  if (cus == 0) {
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      return hipErrorInvalidValue;
+  }
+  // the widest channel tile that divides the layer: 64 x 64 reads each operand
+  // for two blocks; narrower layers share the workgroup's waves over strips
+  if (Cout % 64 == 0 && C1 % 64 == 0 && C2 % 64 == 0)
+    return launch_dw<2, 2, 2, 2>(dY, Cout, X1, C1, X2, C2, dW, db, n, H, W, cus, s);
+  if (Cout % 64 == 0)
+    return launch_dw<2, 1, 4, 1>(dY, Cout, X1, C1, X2, C2, dW, db, n, H, W, cus, s);
+  return launch_dw<1, 1, 4, 1>(dY, Cout, X1, C1, X2, C2, dW, db, n, H, W, 2 * cus, s);
 }
 
 hipError_t unet_conv3_in(const float2* x, const float* w, const float* b, __bf16* Y, int n,
@@ -1265,13 +1439,6 @@ hipError_t unet_up_bwd(const __bf16* gcat, int C1, const __bf16* a, __bf16* ga, 
   const long work = (long)n * H2 * W2 * C;
   hipLaunchKernelGGL(up_bwd_kernel, dim3(blocks(work)), dim3(256), 0, s, gcat, C1, a, ga, n, H2,
                      W2, C);
-  return hipGetLastError();
-}
-
-hipError_t unet_bias_grad(const __bf16* g, float* db, long P, int C, hipStream_t s) {
-  const int ppb = 1024;
-  hipLaunchKernelGGL(bias_grad_kernel, dim3(blocks(P, ppb)), dim3(((C + 63) / 64) * 64), 0, s, g,
-                     db, P, C, ppb);
   return hipGetLastError();
 }
 

@@ -233,3 +233,31 @@ def test_learned_frame_fallback_and_net_paths():
     dphi = d2.last_dphi.cpu().numpy()
     expect = np.angle(z.cpu().numpy())
     assert np.abs(np.angle(np.exp(1j * (dphi - expect)))).max() < 1e-6
+
+
+@pytest.mark.parametrize("levels,base,n,H,W", [
+    (2, 32, 1, 8, 34),    # two rows of strips less than one workgroup; a 2-pixel remainder
+    (2, 32, 3, 24, 130),  # chunks that cross image borders; a strip of 2 pixels in a second block
+    (2, 96, 1, 16, 66),   # channel counts that only 32 divides
+    (3, 64, 2, 16, 260),  # 64-channel tiles on both sources of the decoder convs; 4-row bottom
+])
+def test_gradients_at_strip_and_chunk_edges(levels, base, n, H, W):
+    """The weight-gradient kernels walk 32-pixel strips and chunks of rows
+    across the images of a batch: widths that leave part strips, heights that
+    split unevenly, every channel tile.  Bars as above (the same BF16
+    rounding enters)."""
+    net, ref = _net_and_ref(seed=21, levels=levels, base=base)
+    x, u = _inputs(n, H, W, seed=22)
+    loss = net.loss_grad(torch.from_numpy(x).cuda(), torch.from_numpy(u).cuda())
+    g = net.grads()
+    Lr, gr = U.loss_and_grads(ref, _c2(x), _c2(u), levels)
+    assert abs(loss - Lr) / Lr < 1e-2
+    for k in gr:
+        a, b = g[k].astype(np.float64).ravel(), gr[k].ravel()
+        rel = np.linalg.norm(a - b) / max(np.linalg.norm(b), 1e-30)
+        cos = float(a @ b / max(np.linalg.norm(a) * np.linalg.norm(b), 1e-30))
+        say(f"   {k:8s} rel err {rel:.2e} cos {cos:.5f}")
+        if k.startswith("e0a"):
+            assert rel < 0.2 and cos > 0.98, k
+        else:
+            assert rel < 6e-2, k
