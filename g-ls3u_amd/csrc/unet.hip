@@ -10,6 +10,7 @@
 #include "glsu_internal.h"
 #include "unet_internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -39,6 +40,7 @@ struct Acts {  // activations and gradients for one (n, H, W)
   __bf16 *ge[8], *gea[8], *gp[8], *gd[8], *gda[8], *gcat[8];
   float2* out = nullptr;
   float* loss = nullptr;
+  float* ws = nullptr;  // partial sums of one layer's weight gradient (backward only)
 };
 }  // namespace
 
@@ -163,14 +165,35 @@ static int forward(glsu_unet* h, const float2* x, float2* out, int n, int H, int
   return GLSU_OK;
 }
 
-// loss and gradients (accumulated into zeroed gw/gb) for targets u
+// scratch of the weight gradients: the largest layer's partial sums
+static int grad_ws_alloc(glsu_unet* h, int n, int H, int W) {
+  Acts& a = h->a;
+  if (a.ws) return GLSU_OK;
+  size_t m = 0;
+  for (int l = 0; l < h->levels; ++l) {
+    const int Hl = H >> l, Wl = W >> l, C = h->C(l);
+    m = std::max(m, unet_conv3_dw_floats(C, C, 0, n, Hl, Wl));
+    if (l > 0) m = std::max(m, unet_conv3_dw_floats(C, h->C(l - 1), 0, n, Hl, Wl));
+    if (l + 1 < h->levels) m = std::max(m, unet_conv3_dw_floats(C, C, h->C(l + 1), n, Hl, Wl));
+  }
+  void* p = nullptr;
+  if (hipMalloc(&p, m * sizeof(float)) != hipSuccess)
+    return ufail(GLSU_ERR_DEVICE, "gradient scratch allocation failed");
+  a.bufs.push_back(p);
+  a.ws = (float*)p;
+  return GLSU_OK;
+}
+
+// loss and gradients for targets u
 static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H, int W) {
   Acts& a = h->a;
   const int Lv = h->levels;
   hipStream_t s = h->s;
-  for (auto& l : h->L) {
-    UTRY(unet_fill(l.gw, l.nw(), 0.f, s));
-    UTRY(unet_fill(l.gb, l.cout, 0.f, s));
+  if (int rc = grad_ws_alloc(h, n, H, W)) return rc;
+  // the two layers whose gradients are accumulated; the others are written whole
+  for (Layer* l : {&h->enc(0, 0), &h->out()}) {
+    UTRY(unet_fill(l->gw, l->nw(), 0.f, s));
+    UTRY(unet_fill(l->gb, l->cout, 0.f, s));
   }
   UTRY(unet_fill(a.loss, 1, 0.f, s));
   const long P = (long)n * H * W;
@@ -184,10 +207,10 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
     Layer& la = h->dec(l, 0);
     Layer& lb = h->dec(l, 1);
     const __bf16* low = (l + 1 <= Lv - 2) ? a.d[l + 1] : a.e[Lv - 1];
-    UTRY(unet_conv3_dw(a.gd[l], Cl, a.da[l], Cl, nullptr, 0, lb.gw, lb.gb, n, Hl, Wl, s));
+    UTRY(unet_conv3_dw(a.gd[l], Cl, a.da[l], Cl, nullptr, 0, lb.gw, lb.gb, a.ws, n, Hl, Wl, s));
     UTRY(unet_conv3(a.gd[l], Cl, nullptr, 0, lb.wt, nullptr, a.da[l], a.gda[l], n, Hl, Wl, Cl, 1,
                     s));
-    UTRY(unet_conv3_dw(a.gda[l], Cl, a.e[l], Cl, low, Cn, la.gw, la.gb, n, Hl, Wl, s));
+    UTRY(unet_conv3_dw(a.gda[l], Cl, a.e[l], Cl, low, Cn, la.gw, la.gb, a.ws, n, Hl, Wl, s));
     UTRY(unet_conv3(a.gda[l], Cl, nullptr, 0, la.wt, nullptr, nullptr, a.gcat[l], n, Hl, Wl,
                     Cl + Cn, 1, s));
     __bf16* gl = (l + 1 <= Lv - 2) ? a.gd[l + 1] : a.ge[Lv - 1];
@@ -201,7 +224,7 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
     const int Cl = h->C(l);
     Layer& la = h->enc(l, 0);
     Layer& lb = h->enc(l, 1);
-    UTRY(unet_conv3_dw(a.ge[l], Cl, a.ea[l], Cl, nullptr, 0, lb.gw, lb.gb, n, Hl, Wl, s));
+    UTRY(unet_conv3_dw(a.ge[l], Cl, a.ea[l], Cl, nullptr, 0, lb.gw, lb.gb, a.ws, n, Hl, Wl, s));
     UTRY(unet_conv3(a.ge[l], Cl, nullptr, 0, lb.wt, nullptr, a.ea[l], a.gea[l], n, Hl, Wl, Cl, 1,
                     s));
     if (l == 0) {
@@ -209,7 +232,7 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
       break;
     }
     const int Cp = h->C(l - 1);
-    UTRY(unet_conv3_dw(a.gea[l], Cl, a.p[l - 1], Cp, nullptr, 0, la.gw, la.gb, n, Hl, Wl, s));
+    UTRY(unet_conv3_dw(a.gea[l], Cl, a.p[l - 1], Cp, nullptr, 0, la.gw, la.gb, a.ws, n, Hl, Wl, s));
     UTRY(unet_conv3(a.gea[l], Cl, nullptr, 0, la.wt, nullptr, nullptr, a.gp[l - 1], n, Hl, Wl, Cp,
                     1, s));
     UTRY(unet_pool_bwd(a.e[l - 1], a.gp[l - 1], a.gcat[l - 1], Cp + Cl, a.ge[l - 1], n, H >> (l - 1),

@@ -13,10 +13,12 @@ namespace glsu {
 hipError_t unet_conv3(const __bf16* X1, int C1, const __bf16* X2, int C2, const __bf16* Wt,
                       const float* bias, const __bf16* mask, __bf16* Y, int n, int H, int W,
                       int Cout, int mode, hipStream_t s, __bf16* pool = nullptr);
-// dW [Cout][9][Cin] += weight gradient, db [Cout] += bias gradient (FP32,
-// atomically accumulated)
+// dW [Cout][9][Cin] = weight gradient, db [Cout] = bias gradient (FP32, summed
+// in a fixed order); ws: unet_conv3_dw_floats() floats of scratch
+size_t unet_conv3_dw_floats(int Cout, int C1, int C2, int n, int H, int W);
 hipError_t unet_conv3_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
-                         int C2, float* dW, float* db, int n, int H, int W, hipStream_t s);
+                         int C2, float* dW, float* db, float* ws, int n, int H, int W,
+                         hipStream_t s);
 hipError_t unet_conv3_in(const float2* x, const float* w, const float* b, __bf16* Y, int n,
                          int H, int W, int C0, hipStream_t s);
 hipError_t unet_conv3_in_dw(const float2* x, const __bf16* dY, float* dW, float* db, int n,

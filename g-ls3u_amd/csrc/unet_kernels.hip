@@ -779,8 +779,11 @@ __global__ __launch_bounds__(512, 1) void conv3_res64_kernel(
 // each); R rows are staged at a time, double-buffered, the next rows' global
 // loads in flight during the MFMAs.  The rows of all images are one sequence
 // with a zero row after each image (img * (H + 1) + y), cut into chunks, one
-// per workgroup, so the launch fills the chip whatever n, H and W are; strips
-// are summed through LDS and chunks by FP32 atomics.
+// per workgroup, so the launch fills the chip whatever n, H and W are.  The
+// strips of a workgroup are summed through LDS; every workgroup stores its sum
+// as one partial (in accumulator order, 256-byte runs) and dw_reduce_kernel
+// adds the partials in a fixed order and writes the gradients: FP32 atomics on
+// the shared gradient from every workgroup took longer than the MFMAs.
 // Bound at full resolution (32 channels) by memory, above it by LDS reads
 // (16 transposing reads per 36 MFMAs) and the MFMAs.
 constexpr int kGrStrip = 32;
@@ -807,21 +810,21 @@ struct GradConv {
   static constexpr int XSlots = XW * NB * 4, YSlots = YW * MB * 4;  // 16-byte slots of a row
   static constexpr int XLd = (XSlots + Threads - 1) / Threads;
   static constexpr int YLd = (YSlots + Threads - 1) / Threads;
+  static constexpr int Blocks = MB * NB;             // 32 x 32 blocks of a tile
   // strip sums go through LDS, one tap at a time, after the main loop
-  static_assert(S == 1 || MB * NB * (S - 1) * 4096 <= 2 * Stage * 2, "strip sums fit the stages");
+  static_assert(MB * NB * (S - 1) * 4096 <= 2 * Stage * 2, "strip sums fit the stages");
 };
 
 template <int MB, int NB, int S, int R>
-__global__ __launch_bounds__(64 * MB * NB * S) void conv3_dw_kernel(
+__global__ __launch_bounds__(64 * MB * NB * S, 2) void conv3_dw_kernel(
     const __bf16* __restrict__ dY, int Cout, const __bf16* __restrict__ X1, int C1,
-    const __bf16* __restrict__ X2, int C2, float* __restrict__ dW, float* __restrict__ db, int n,
-    int H, int W, int rows_per_wg) {
+    const __bf16* __restrict__ X2, int C2, float* __restrict__ part, int n, int H, int W,
+    int rows_per_wg, int strips_per_wg) {
   using G = GradConv<MB, NB, S, R>;
   __shared__ __attribute__((aligned(16))) __bf16 sm[2][G::Stage];
   const int Cin = C1 + C2;
   const int ncx = Cin / (32 * NB);
   const int co0 = (blockIdx.y / ncx) * 32 * MB, ci0 = (blockIdx.y % ncx) * 32 * NB;
-  const int x0 = blockIdx.z * kGrStrip * S;
   const int V = n * (H + 1);  // rows of all images, each followed by a zero row
   const int v0 = blockIdx.x * rows_per_wg, v1 = min(V, v0 + rows_per_wg);
   const int tid = threadIdx.x, wave = tid / 64, lane = tid % 64;
@@ -835,18 +838,21 @@ __global__ __launch_bounds__(64 * MB * NB * S) void conv3_dw_kernel(
   // offset, and whether the pixel is in the image
   int xo[G::XLd], yo[G::YLd];
   unsigned xin = 0, yin = 0;
+  auto slots = [&](int x0) {
+    xin = yin = 0;
 #pragma unroll
-  for (int k = 0; k < G::XLd; ++k) {
-    const int i = tid + G::Threads * k, px = i / (NB * 4), g = i % (NB * 4), x = x0 - 1 + px;
-    xin |= (x >= 0 && x < W ? 1u : 0u) << k;
-    xo[k] = (min(max(x, 0), W - 1) >> sh) * Cx + g * 8;
-  }
+    for (int k = 0; k < G::XLd; ++k) {
+      const int i = tid + G::Threads * k, px = i / (NB * 4), g = i % (NB * 4), x = x0 - 1 + px;
+      xin |= (x >= 0 && x < W ? 1u : 0u) << k;
+      xo[k] = (min(max(x, 0), W - 1) >> sh) * Cx + g * 8;
+    }
 #pragma unroll
-  for (int k = 0; k < G::YLd; ++k) {
-    const int i = tid + G::Threads * k, px = i / (MB * 4), g = i % (MB * 4), x = x0 + px;
-    yin |= (x < W ? 1u : 0u) << k;
-    yo[k] = min(x, W - 1) * Cout + co0 + g * 8;
-  }
+    for (int k = 0; k < G::YLd; ++k) {
+      const int i = tid + G::Threads * k, px = i / (MB * 4), g = i % (MB * 4), x = x0 + px;
+      yin |= (x < W ? 1u : 0u) << k;
+      yo[k] = min(x, W - 1) * Cout + co0 + g * 8;
+    }
+  };
   bf16x8 lx[R][G::XLd], ly[R][G::YLd];
   // input rows v .. v + R - 1 and the dY rows one below them
   auto load = [&](int v) {
@@ -901,8 +907,6 @@ __global__ __launch_bounds__(64 * MB * NB * S) void conv3_dw_kernel(
   bf16x8 a0[2], a1[2], a2[2], ones;  // dY rows vi - 1, vi, vi + 1
 #pragma unroll
   for (int i = 0; i < 8; ++i) ones[i] = (__bf16)1.f;
-#pragma unroll
-  for (int i = 0; i < 2; ++i) a1[i] = a2[i] = zero8();
   const bool bias = ci0 == 0 && wn == 0;
   // transposing read: lane l of a 16-lane group addresses pixel l / 4, channels
   // 4 (l % 4) .. + 3, and receives channel l of the four pixels; group lk reads
@@ -911,84 +915,137 @@ __global__ __launch_bounds__(64 * MB * NB * S) void conv3_dw_kernel(
   const int xbase = (kGrStrip * s + lpx) * G::XP + wn * 32 + lch;
   const int ybase = (kGrStrip * s + lpx) * G::YP + wm * 32 + lch;
 
-  load(v0 - 1);
-  store(sm[0]);
-  __syncthreads();
-  int cur = 0;
-  for (int v = v0 - 1; v <= v1; v += R, cur ^= 1) {
-    const bool more = v + R <= v1;
-    if (more) load(v + R);
+  const int strips = (W + kGrStrip * S - 1) / (kGrStrip * S);
+  const int z1 = min(strips, ((int)blockIdx.z + 1) * strips_per_wg);
+  for (int z = blockIdx.z * strips_per_wg; z < z1; ++z) {
+    slots(z * kGrStrip * S);
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const __bf16* bx = sm[cur] + r * (G::XRow + G::YRow) + xbase;
-      const __bf16* by = sm[cur] + r * (G::XRow + G::YRow) + G::XRow + ybase;
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        a0[i] = a1[i];
-        a1[i] = a2[i];
-        a2[i] = lds_tr8(by + i * 16, by + i * 16 + 16 * G::YP);
-      }
-      if (bias) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-          accb[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[i], ones, accb[i], 0, 0, 0);
-      }
-#pragma unroll
-      for (int dx = 0; dx < 3; ++dx) {
-        bf16x8 b[2];
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-          b[j] = lds_tr8(bx + dx * G::XP + j * 16, bx + (dx + 16) * G::XP + j * 16);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-#pragma unroll
-          for (int j = 0; j < 2; ++j) {
-            // output row one below, at and above the input row: tap rows 0, 1, 2
-            acc[dx][i][j] =
-                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[i], b[j], acc[dx][i][j], 0, 0, 0);
-            acc[3 + dx][i][j] =
-                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[i], b[j], acc[3 + dx][i][j], 0, 0, 0);
-            acc[6 + dx][i][j] =
-                __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[i], b[j], acc[6 + dx][i][j], 0, 0, 0);
-          }
-      }
-    }
-    if (more) store(sm[cur ^ 1]);
+    for (int i = 0; i < 2; ++i) a1[i] = a2[i] = zero8();
+    load(v0 - 1);
+    store(sm[0]);
     __syncthreads();
-  }
-  // acc[t][i][j][r]: co = co0 + 32 wm + 16 i + 4 lk + r, ci = ci0 + 32 wn + 16 j + lr
-  const int lr = lane % 16, lk = lane / 16;
-  float* red = (float*)&sm[0][0];
-  const int blk = wave % (MB * NB);
+    int cur = 0;
+    for (int v = v0 - 1; v <= v1; v += R, cur ^= 1) {
+      const bool more = v + R <= v1;
+      if (more) load(v + R);
 #pragma unroll
-  for (int t = 0; t < 9; ++t) {
-    if constexpr (S > 1) {
-      if (s > 0) {
-        float* o = red + ((s - 1) * MB * NB + blk) * 1024 + lane;
+      for (int r = 0; r < R; ++r) {
+        const __bf16* bx = sm[cur] + r * (G::XRow + G::YRow) + xbase;
+        const __bf16* by = sm[cur] + r * (G::XRow + G::YRow) + G::XRow + ybase;
 #pragma unroll
-        for (int k = 0; k < 16; ++k) o[64 * k] = acc[t][k / 8][(k / 4) % 2][k % 4];
+        for (int i = 0; i < 2; ++i) {
+          a0[i] = a1[i];
+          a1[i] = a2[i];
+          a2[i] = lds_tr8(by + i * 16, by + i * 16 + 16 * G::YP);
+        }
+        if (bias) {
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+            accb[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[i], ones, accb[i], 0, 0, 0);
+        }
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx) {
+          bf16x8 b[2];
+#pragma unroll
+          for (int j = 0; j < 2; ++j)
+            b[j] = lds_tr8(bx + dx * G::XP + j * 16, bx + (dx + 16) * G::XP + j * 16);
+#pragma unroll
+          for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+              // output row one below, at and above the input row: tap rows 0, 1, 2
+              acc[dx][i][j] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(a2[i], b[j], acc[dx][i][j], 0, 0, 0);
+              acc[3 + dx][i][j] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(a1[i], b[j], acc[3 + dx][i][j], 0, 0, 0);
+              acc[6 + dx][i][j] =
+                  __builtin_amdgcn_mfma_f32_16x16x32_bf16(a0[i], b[j], acc[6 + dx][i][j], 0, 0, 0);
+            }
+        }
       }
+      if (more) store(sm[cur ^ 1]);
       __syncthreads();
     }
+  }
+  // acc[t][i][j][r]: co = co0 + 32 wm + 16 i + 4 lk + r, ci = ci0 + 32 wn + 16 j + lr;
+  // partial: [tile][block][tap][16 registers][lane], then the biases [Cout]
+  const int lr = lane % 16, lk = lane / 16;
+  float* red = (float*)&sm[0][0];
+  const int blk = wave % G::Blocks;
+  const size_t pstride = (size_t)Cout * 9 * Cin + Cout;
+  part += ((size_t)blockIdx.z * gridDim.x + blockIdx.x) * pstride;
+  float* out = part + ((size_t)blockIdx.y * G::Blocks + blk) * 9 * 1024 + lane;
+#pragma unroll
+  for (int t = 0; t < 9; ++t) {
+    if (s > 0) {
+      float* o = red + ((s - 1) * G::Blocks + blk) * 1024 + lane;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) o[64 * k] = acc[t][k / 8][(k / 4) % 2][k % 4];
+    }
+    __syncthreads();
     if (s == 0) {
 #pragma unroll
       for (int k = 0; k < 16; ++k) {
-        const int i = k / 8, j = (k / 4) % 2, r = k % 4;
-        float v = acc[t][i][j][r];
+        float v = acc[t][k / 8][(k / 4) % 2][k % 4];
 #pragma unroll
-        for (int q = 0; q < S - 1; ++q) v += red[(q * MB * NB + blk) * 1024 + 64 * k + lane];
-        const int co = co0 + 32 * wm + 16 * i + 4 * lk + r, ci = ci0 + 32 * wn + 16 * j + lr;
-        atomicAdd(dW + ((size_t)co * 9 + t) * Cin + ci, v);
+        for (int q = 0; q < S - 1; ++q) v += red[(q * G::Blocks + blk) * 1024 + 64 * k + lane];
+        out[(16 * t + k) * 64] = v;
       }
     }
-    if constexpr (S > 1) __syncthreads();
+    __syncthreads();
   }
-  if (bias && lr == 0) {
+  if (ci0 == 0) {
+    if (bias && lr == 0) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+      for (int k = 0; k < 8; ++k)
+        red[s * 32 * MB + 32 * wm + 16 * (k / 4) + 4 * lk + k % 4] = accb[k / 4][k % 4];
+    }
+    __syncthreads();
+    if (tid < 32 * MB) {
+      float v = 0.f;
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        atomicAdd(db + co0 + 32 * wm + 16 * i + 4 * lk + r, accb[i][r]);
+      for (int q = 0; q < S; ++q) v += red[q * 32 * MB + tid];
+      part[(size_t)Cout * 9 * Cin + co0 + tid] = v;
+    }
+  }
+}
+
+// Sum of np partials of conv3_dw_kernel<MB, NB, ...>, four consecutive values
+// per thread: 16 threads read a partial's 256-byte run, 16 slices of partials
+// per workgroup run side by side (the number of values alone would leave most
+// CUs idle: 9 k for a 32 x 32 layer) and meet in LDS.
+template <int MB, int NB>
+__global__ __launch_bounds__(256) void dw_reduce_kernel(const float* __restrict__ part, int np,
+                                                        float* __restrict__ dW,
+                                                        float* __restrict__ db, int Cout,
+                                                        int Cin) {
+  __shared__ floatx4 red[16][16];
+  const long nw = (long)Cout * 9 * Cin, count = nw + Cout;
+  const int col = threadIdx.x % 16, slice = threadIdx.x / 16;
+  const long i = ((long)blockIdx.x * 16 + col) * 4;
+  floatx4 v{0.f, 0.f, 0.f, 0.f};
+  if (i < count) {
+#pragma unroll 4
+    for (int p = slice; p < np; p += 16) v += *(const floatx4*)(part + p * (size_t)count + i);
+  }
+  red[slice][col] = v;
+  __syncthreads();
+  if (slice != 0 || i >= count) return;
+#pragma unroll
+  for (int q = 1; q < 16; ++q) v += red[q][col];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const long e = i + j;
+    if (e >= nw) {
+      db[e - nw] = v[j];
+      continue;
+    }
+    const int lane = (int)(e % 64), k = (int)(e / 64 % 16), t = (int)(e / 1024 % 9);
+    const int b = (int)(e / 9216), blk = b % (MB * NB), tile = b / (MB * NB);
+    const int ncx = Cin / (32 * NB);
+    const int co = ((tile / ncx) * MB + blk / NB) * 32 + 16 * (k / 8) + 4 * (lane / 16) + k % 4;
+    const int ci = ((tile % ncx) * NB + blk % NB) * 32 + 16 * ((k / 4) % 2) + lane % 16;
+    dW[((size_t)co * 9 + t) * Cin + ci] = v[j];
   }
 }
 
@@ -1351,40 +1408,88 @@ hipError_t unet_conv3(const __bf16* X1, int C1, const __bf16* X2, int C2, const 
   return unet_maxpool2(Y, pool, n, H, W, Cout, s);
 }
 
+// Partition of one weight gradient: workgroups per (co, ci) tile along the
+// rows and along the strips; their product is the number of partials.
+struct DwSplit {
+  int rows, chunks, strips, groups;  // rows per chunk, chunks, strips per group, groups
+};
+template <int MB, int NB, int S, int R>
+static DwSplit dw_split(int Cout, int Cin, int n, int H, int W, int wgs) {
+  const int tiles = (Cout / (32 * MB)) * (Cin / (32 * NB));
+  const int ns = (W + kGrStrip * S - 1) / (kGrStrip * S);
+  // as many partials as fill the chip once, but at least six rows each (every
+  // chunk reads two input rows more than it owns)
+  const int want = std::max(1, wgs / tiles), V = n * (H + 1);
+  DwSplit d;
+  const int g = std::min(ns, want);
+  d.strips = (ns + g - 1) / g;
+  d.groups = (ns + d.strips - 1) / d.strips;
+  const int c = std::max(1, std::min(want / d.groups, V / 6));
+  d.rows = (V + c - 1) / c;
+  d.chunks = (V + d.rows - 1) / d.rows;
+  return d;
+}
 template <int MB, int NB, int S, int R>
 static hipError_t launch_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
-                            int C2, float* dW, float* db, int n, int H, int W, int wgs,
+                            int C2, float* dW, float* db, float* ws, int n, int H, int W, int wgs,
                             hipStream_t s) {
-  using G = GradConv<MB, NB, S, R>;
-  const int tiles = (Cout / (32 * MB)) * ((C1 + C2) / (32 * NB));
-  const int strips = (W + kGrStrip * S - 1) / (kGrStrip * S);
-  // chunks of rows: as many as fill the chip once, but at least six rows each
-  // (every chunk reads two input rows more than it owns)
-  const int V = n * (H + 1);
-  const int chunks = std::max(1, std::min(wgs / std::max(1, tiles * strips), V / 6));
-  const int rows = (V + chunks - 1) / chunks;
-  hipLaunchKernelGGL((conv3_dw_kernel<MB, NB, S, R>), dim3((V + rows - 1) / rows, tiles, strips),
-                     dim3(G::Threads), 0, s, dY, Cout, X1, C1, X2, C2, dW, db, n, H, W, rows);
+  const int Cin = C1 + C2, tiles = (Cout / (32 * MB)) * (Cin / (32 * NB));
+  const DwSplit d = dw_split<MB, NB, S, R>(Cout, Cin, n, H, W, wgs);
+  hipLaunchKernelGGL((conv3_dw_kernel<MB, NB, S, R>), dim3(d.chunks, tiles, d.groups),
+                     dim3(GradConv<MB, NB, S, R>::Threads), 0, s, dY, Cout, X1, C1, X2, C2, ws, n,
+                     H, W, d.rows, d.strips);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  const long count = (long)Cout * 9 * Cin + Cout;
+  hipLaunchKernelGGL((dw_reduce_kernel<MB, NB>), dim3(blocks(count, 64)), dim3(256), 0, s, ws,
+                     d.chunks * d.groups, dW, db, Cout, Cin);
   return hipGetLastError();
 }
 
-hipError_t unet_conv3_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
-                         int C2, float* dW, float* db, int n, int H, int W, hipStream_t s) {
-  if ((C1 % 32) || (C2 % 32) || (Cout % 32) || (C2 && ((H | W) & 1))) return hipErrorInvalidValue;
+static int device_cus() {
   static int cus = 0;
   if (cus == 0) {
-    int dev = 0;
+    int dev = 0, v = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      return hipErrorInvalidValue;
+        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      return 0;
+    cus = v;
   }
-  // the widest channel tile that divides the layer: 64 x 64 reads each operand
-  // for two blocks; narrower layers share the workgroup's waves over strips
-  if (Cout % 64 == 0 && C1 % 64 == 0 && C2 % 64 == 0)
-    return launch_dw<2, 2, 2, 2>(dY, Cout, X1, C1, X2, C2, dW, db, n, H, W, cus, s);
-  if (Cout % 64 == 0)
-    return launch_dw<2, 1, 4, 1>(dY, Cout, X1, C1, X2, C2, dW, db, n, H, W, cus, s);
-  return launch_dw<1, 1, 4, 1>(dY, Cout, X1, C1, X2, C2, dW, db, n, H, W, 2 * cus, s);
+  return cus;
+}
+
+// The widest channel tile that divides the layer: 64 x 64 reads each operand
+// for two blocks; narrower layers share the workgroup's waves over strips.
+static int dw_tile(int Cout, int C1, int C2) {
+  if (Cout % 64) return 0;
+  return C1 % 64 || C2 % 64 ? 1 : 2;
+}
+
+size_t unet_conv3_dw_floats(int Cout, int C1, int C2, int n, int H, int W) {
+  const int cus = std::max(1, device_cus()), Cin = C1 + C2;
+  DwSplit d;
+  switch (dw_tile(Cout, C1, C2)) {
+    case 2: d = dw_split<2, 2, 2, 2>(Cout, Cin, n, H, W, cus); break;
+    case 1: d = dw_split<2, 1, 4, 1>(Cout, Cin, n, H, W, cus); break;
+    default: d = dw_split<1, 1, 4, 1>(Cout, Cin, n, H, W, 2 * cus); break;
+  }
+  return (size_t)d.chunks * d.groups * ((size_t)Cout * 9 * Cin + Cout);
+}
+
+hipError_t unet_conv3_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
+                         int C2, float* dW, float* db, float* ws, int n, int H, int W,
+                         hipStream_t s) {
+  if ((C1 % 32) || (C2 % 32) || (Cout % 32) || (C2 && ((H | W) & 1))) return hipErrorInvalidValue;
+  const int cus = device_cus();
+  if (cus < 1) return hipErrorInvalidValue;
+  switch (dw_tile(Cout, C1, C2)) {
+    case 2:
+      return launch_dw<2, 2, 2, 2>(dY, Cout, X1, C1, X2, C2, dW, db, ws, n, H, W, cus, s);
+    case 1:
+      return launch_dw<2, 1, 4, 1>(dY, Cout, X1, C1, X2, C2, dW, db, ws, n, H, W, cus, s);
+    default:
+      return launch_dw<1, 1, 4, 1>(dY, Cout, X1, C1, X2, C2, dW, db, ws, n, H, W, 2 * cus, s);
+  }
 }
 
 hipError_t unet_conv3_in(const float2* x, const float* w, const float* b, __bf16* Y, int n,
