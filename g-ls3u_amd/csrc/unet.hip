@@ -169,7 +169,8 @@ static int forward(glsu_unet* h, const float2* x, float2* out, int n, int H, int
 static int grad_ws_alloc(glsu_unet* h, int n, int H, int W) {
   Acts& a = h->a;
   if (a.ws) return GLSU_OK;
-  size_t m = 0;
+  size_t m = std::max(unet_conv3_in_dw_floats(n, H, h->C(0)),
+                      unet_conv1_out_bwd_floats((long)n * H * W, h->C(0)));
   for (int l = 0; l < h->levels; ++l) {
     const int Hl = H >> l, Wl = W >> l, C = h->C(l);
     m = std::max(m, unet_conv3_dw_floats(C, C, 0, n, Hl, Wl));
@@ -190,15 +191,10 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
   const int Lv = h->levels;
   hipStream_t s = h->s;
   if (int rc = grad_ws_alloc(h, n, H, W)) return rc;
-  // the two layers whose gradients are accumulated; the others are written whole
-  for (Layer* l : {&h->enc(0, 0), &h->out()}) {
-    UTRY(unet_fill(l->gw, l->nw(), 0.f, s));
-    UTRY(unet_fill(l->gb, l->cout, 0.f, s));
-  }
-  UTRY(unet_fill(a.loss, 1, 0.f, s));
   const long P = (long)n * H * W;
   Layer& o = h->out();
-  UTRY(unet_conv1_out_bwd(a.d[0], a.out, u, o.w, a.gd[0], o.gw, o.gb, a.loss, P, h->C(0), s));
+  UTRY(unet_conv1_out_bwd(a.d[0], a.out, u, o.w, a.gd[0], o.gw, o.gb, a.loss, a.ws, P,
+                          h->C(0), s));
   // decoder, top level first; gd[l]: gradient at the pre-activation of d_l
   __bf16* ge_top = nullptr;
   for (int l = 0; l <= Lv - 2; ++l) {
@@ -228,7 +224,7 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
     UTRY(unet_conv3(a.ge[l], Cl, nullptr, 0, lb.wt, nullptr, a.ea[l], a.gea[l], n, Hl, Wl, Cl, 1,
                     s));
     if (l == 0) {
-      UTRY(unet_conv3_in_dw(x, a.gea[0], la.gw, la.gb, n, H, W, Cl, s));
+      UTRY(unet_conv3_in_dw(x, a.gea[0], la.gw, la.gb, a.ws, n, H, W, Cl, s));
       break;
     }
     const int Cp = h->C(l - 1);

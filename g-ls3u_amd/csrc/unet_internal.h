@@ -21,13 +21,16 @@ hipError_t unet_conv3_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, c
                          hipStream_t s);
 hipError_t unet_conv3_in(const float2* x, const float* w, const float* b, __bf16* Y, int n,
                          int H, int W, int C0, hipStream_t s);
-hipError_t unet_conv3_in_dw(const float2* x, const __bf16* dY, float* dW, float* db, int n,
-                            int H, int W, int C0, hipStream_t s);
+// input and output layer gradients, written whole; ws: *_floats() of scratch
+size_t unet_conv3_in_dw_floats(int n, int H, int C0);
+hipError_t unet_conv3_in_dw(const float2* x, const __bf16* dY, float* dW, float* db, float* ws,
+                            int n, int H, int W, int C0, hipStream_t s);
 hipError_t unet_conv1_out(const __bf16* d, const float2* x, const float* w, const float* b,
                           float2* out, long P, int C0, hipStream_t s);
 hipError_t unet_conv1_out_bwd(const __bf16* d, const float2* out, const float2* u,
                               const float* w, __bf16* dd, float* dW, float* db, float* loss,
-                              long P, int C0, hipStream_t s);
+                              float* ws, long P, int C0, hipStream_t s);
+size_t unet_conv1_out_bwd_floats(long P, int C0);
 hipError_t unet_maxpool2(const __bf16* x, __bf16* y, int n, int H, int W, int C, hipStream_t s);
 hipError_t unet_pool_bwd(const __bf16* e, const __bf16* gp, const __bf16* gskip, int Cs,
                          __bf16* ge, int n, int H, int W, int C, hipStream_t s);
@@ -37,6 +40,5 @@ hipError_t unet_adam(float* w, const float* g, float* m, float* v, long count, f
                      float b1, float b2, float eps, int step, hipStream_t s);
 hipError_t unet_weights_bf16(const float* w, __bf16* wf, __bf16* wt, int Cout, int Cin,
                              hipStream_t s);
-hipError_t unet_fill(float* p, long count, float v, hipStream_t s);
 
 }  // namespace glsu

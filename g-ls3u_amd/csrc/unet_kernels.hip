@@ -1091,36 +1091,115 @@ __global__ __launch_bounds__(256) void conv3_in_kernel(const float2* __restrict_
   }
 }
 
-// weight/bias gradient of the input layer: dW[co][t][c] = sum_p dY[p][co] x[p+off_t][c]
-__global__ __launch_bounds__(1024) void conv3_in_dw_kernel(const float2* __restrict__ x,
-                                                          const __bf16* __restrict__ dY,
-                                                          float* __restrict__ dW,
-                                                          float* __restrict__ db, int n, int H,
-                                                          int W, int C0, int pix_per_block) {
-  // thread k < C0*19 (k over blockIdx.y, threadIdx.x) owns one weight (or
-  // bias) and sums it over the block's pixels
-  const int k = blockIdx.y * blockDim.x + threadIdx.x;
-  const long P = (long)n * H * W;
-  const long p0 = (long)blockIdx.x * pix_per_block, p1 = std::min(P, p0 + pix_per_block);
-  if (k >= C0 * 19) return;
-  const bool isb = k >= C0 * 18;
-  const int co = isb ? k - C0 * 18 : k / 18;
-  const int t = (k % 18) / 2, c = k % 2;
-  float s = 0.f;
-  for (long p = p0; p < p1; ++p) {
-    const float g = (float)dY[(size_t)p * C0 + co];
-    if (isb) {
-      s += g;
-      continue;
+// One halving step per lane bit (from bit O down to 1) of a sum over the
+// wave's lanes of N values each: the lanes with the bit set keep the upper
+// half (rounded up) of the values, the others the lower.  `at` collects the
+// index of the lane's first remaining value, `cnt` how many it has (an odd
+// count leaves the upper half one short).
+template <int N, int O>
+__device__ __forceinline__ void lane_fold(float* v, int lane, int& at, int& cnt) {
+  constexpr int M = (N + 1) / 2;
+  const bool up = lane & O;
+#pragma unroll
+  for (int i = 0; i < M; ++i) {
+    const float hi = i + M < N ? v[i + M] : 0.f;
+    const float keep = up ? hi : v[i], give = up ? v[i] : hi;
+    v[i] = keep + __shfl_xor(give, O);
+  }
+  at += up ? M : 0;
+  cnt = up ? max(cnt - M, 0) : min(cnt, M);
+  if constexpr (O > 1) lane_fold<M, O / 2>(v, lane, at, cnt);
+}
+
+// weight/bias gradient of the input layer: dW[co][t][c] = sum_p dY[p][co]
+// x[p+off_t][c].  FP32 on the vector ALU (x stays FP32).  A lane walks pixels
+// of its row with 4 channels x (18 weights + bias) sums in registers: 76 FMAs
+// on 9 + 1 loads, against two loads per FMA with one thread per weight (8
+// channels a lane spill at two waves per SIMD).  The eight waves of a
+// workgroup take the eight 4-channel groups of 32 channels, so together they
+// read whole lines of dY.  A wave's sums meet through lane swaps at the
+// end and go out as one partial per workgroup (partials_kernel adds them:
+// atomics on the 608 shared sums serialised).  Bound by the FMAs (16 us at 1 M pixels
+// and 32 channels) and the 72 MB read.
+__global__ __launch_bounds__(512, 4) void conv3_in_dw_kernel(const float2* __restrict__ x,
+                                                             const __bf16* __restrict__ dY,
+                                                             float* __restrict__ part, int n,
+                                                             int H, int W, int C0) {
+  const int lane = threadIdx.x % 64, co = blockIdx.y * 32 + (threadIdx.x / 64) * 4;
+  const int rows = n * H;
+  float acc[4][19];
+#pragma unroll
+  for (int k = 0; k < 4; ++k)
+#pragma unroll
+    for (int i = 0; i < 19; ++i) acc[k][i] = 0.f;
+  for (int r = blockIdx.x; r < rows; r += gridDim.x) {
+    const int y = r % H;  // the row's image starts at row r - y
+    const float2* xr[3];
+    bool up[3];
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const int y2 = y + d - 1;
+      up[d] = y2 >= 0 && y2 < H;
+      xr[d] = x + (size_t)(r - y + min(max(y2, 0), H - 1)) * W;
     }
-    const int xx = (int)(p % W), yy = (int)((p / W) % H), img = (int)(p / ((long)W * H));
-    const int y2 = yy + t / 3 - 1, x2 = xx + t % 3 - 1;
-    if (y2 >= 0 && y2 < H && x2 >= 0 && x2 < W) {
-      const float2 v = x[((size_t)img * H + y2) * W + x2];
-      s = fmaf(g, c ? v.y : v.x, s);
+    for (int xx = lane; xx < W; xx += 64) {
+      float in[18];
+#pragma unroll
+      for (int t = 0; t < 9; ++t) {
+        const int x2 = xx + t % 3 - 1;
+        const float2 v = xr[t / 3][min(max(x2, 0), W - 1)];
+        const bool inside = up[t / 3] && x2 >= 0 && x2 < W;
+        in[2 * t] = inside ? v.x : 0.f;
+        in[2 * t + 1] = inside ? v.y : 0.f;
+      }
+      const bf16x4 g4 = *(const bf16x4*)(dY + ((size_t)r * W + xx) * C0 + co);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const float g = (float)g4[k];
+#pragma unroll
+        for (int i = 0; i < 18; ++i) acc[k][i] = fmaf(g, in[i], acc[k][i]);
+        acc[k][18] += g;
+      }
     }
   }
-  atomicAdd(isb ? db + co : dW + k, s);
+  // sum over the wave's lanes by halving: at each step a lane hands half of its
+  // values to its partner and adds the partner's share of the other half (77
+  // exchanges for 76 sums instead of six each)
+  float v[76];
+#pragma unroll
+  for (int i = 0; i < 76; ++i) v[i] = acc[i / 19][i % 19];
+  int at = 0, cnt = 76;
+  lane_fold<76, 32>(v, lane, at, cnt);
+  part += (size_t)blockIdx.x * C0 * 19;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const int i = at + q, k = i / 19, w = i % 19;
+    if (q < cnt) part[w == 18 ? C0 * 18 + co + k : (co + k) * 18 + w] = v[q];
+  }
+}
+
+// out0[n0], out1[n1], out2[n2] = the sums over np partials of n0 + n1 + n2
+// consecutive values (pitch floats apart), in a fixed order: 16 values side by
+// side, 16 slices of partials per workgroup.
+__global__ __launch_bounds__(256) void partials_kernel(const float* __restrict__ part, int np,
+                                                       int pitch, float* __restrict__ out0, int n0,
+                                                       float* __restrict__ out1, int n1,
+                                                       float* __restrict__ out2, int n2) {
+  __shared__ float red[16][17];
+  const int col = threadIdx.x % 16, slice = threadIdx.x / 16, i = blockIdx.x * 16 + col;
+  float v = 0.f;
+  if (i < n0 + n1 + n2) {
+#pragma unroll 8
+    for (int p = slice; p < np; p += 16) v += part[(size_t)p * pitch + i];
+  }
+  red[slice][col] = v;
+  __syncthreads();
+  if (slice != 0 || i >= n0 + n1 + n2) return;
+#pragma unroll
+  for (int q = 1; q < 16; ++q) v += red[q][col];
+  if (i < n0) out0[i] = v;
+  else if (i < n0 + n1) out1[i - n0] = v;
+  else out2[i - n0 - n1] = v;
 }
 
 // ------------------------------------------------------------------------
@@ -1148,65 +1227,64 @@ __global__ __launch_bounds__(256) void conv1_out_kernel(const __bf16* __restrict
 
 // Loss L = mean |out - u|^2 and its backward through the output layer:
 // g = 2 (out - u) / P; dd = (W^T g) * (d > 0); dW += g d^T; db += g.
-// Per-block partial sums of the loss and of dW/db go out through atomics.
+// Four threads per pixel, 8 channels each (32 channels per blockIdx.y), so d
+// and dd move in 16-byte pieces of whole lines; every thread keeps its 16
+// weight sums (and the loss and bias sums) in registers over a grid-stride
+// walk and the workgroup reduces once at the end, instead of a workgroup-wide
+// reduction per channel for every 256 pixels; partials_kernel adds the
+// workgroups' partials (atomics on the 67 shared sums serialised: more
+// workgroups made the kernel slower).  Bound by memory: 144 MB at 1 M
+// pixels and 32 channels.
 __global__ __launch_bounds__(256) void conv1_out_bwd_kernel(
     const __bf16* __restrict__ d, const float2* __restrict__ out, const float2* __restrict__ u,
-    const float* __restrict__ w, __bf16* __restrict__ dd, float* __restrict__ dW,
-    float* __restrict__ db, float* __restrict__ loss, long P, int C0) {
-  extern __shared__ float red[];  // (2*C0 + 3) x 256 partials would be large: reduce per warp
-  const long p = (long)blockIdx.x * blockDim.x + threadIdx.x;
+    const float* __restrict__ w, __bf16* __restrict__ dd, float* __restrict__ part, long P,
+    int C0) {
+  __shared__ float red[4][4][19];  // [wave][channel group][sum]
+  const int g = threadIdx.x % 4, lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  const int c0 = blockIdx.y * 32 + 8 * g;
   const float invP = 1.f / (float)P;
-  float g0 = 0.f, g1 = 0.f, l = 0.f;
-  if (p < P) {
+  float w0[8], w1[8], s[19];  // s: dW[0][8], dW[1][8], loss, db[0], db[1]
+#pragma unroll
+  for (int k = 0; k < 8; ++k) {
+    w0[k] = w[c0 + k];
+    w1[k] = w[C0 + c0 + k];
+  }
+#pragma unroll
+  for (int k = 0; k < 19; ++k) s[k] = 0.f;
+  for (long p = (long)blockIdx.x * 64 + threadIdx.x / 4; p < P; p += (long)gridDim.x * 64) {
     const float2 o = out[p], t = u[p];
+    const bf16x8 v = *(const bf16x8*)(d + (size_t)p * C0 + c0);
     const float r0 = o.x - t.x, r1 = o.y - t.y;
-    l = (r0 * r0 + r1 * r1) * invP;
-    g0 = 2.f * r0 * invP;
-    g1 = 2.f * r1 * invP;
-  }
-  // loss and bias gradients: block reduction
-  float* s = red;
-  s[threadIdx.x] = l;
-  s[256 + threadIdx.x] = g0;
-  s[512 + threadIdx.x] = g1;
-  __syncthreads();
-  for (int o = 128; o > 0; o >>= 1) {
-    if ((int)threadIdx.x < o) {
-      s[threadIdx.x] += s[threadIdx.x + o];
-      s[256 + threadIdx.x] += s[256 + threadIdx.x + o];
-      s[512 + threadIdx.x] += s[512 + threadIdx.x + o];
+    const float g0 = 2.f * r0 * invP, g1 = 2.f * r1 * invP;
+    s[16] += (r0 * r0 + r1 * r1) * invP;
+    s[17] += g0;
+    s[18] += g1;
+    bf16x8 q;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float f = (float)v[k];
+      q[k] = (__bf16)(f > 0.f ? w0[k] * g0 + w1[k] * g1 : 0.f);
+      s[k] = fmaf(g0, f, s[k]);
+      s[8 + k] = fmaf(g1, f, s[8 + k]);
     }
-    __syncthreads();
+    *(bf16x8*)(dd + (size_t)p * C0 + c0) = q;
   }
-  if (threadIdx.x == 0) {
-    atomicAdd(loss, s[0]);
-    atomicAdd(db, s[256]);
-    atomicAdd(db + 1, s[512]);
+#pragma unroll
+  for (int k = 0; k < 19; ++k) {
+    float v = s[k];
+#pragma unroll
+    for (int o = 32; o >= 4; o >>= 1) v += __shfl_xor(v, o);
+    if (lane < 4) red[wave][lane][k] = v;
   }
   __syncthreads();
-  // per channel: dd and the dW partial (block-reduced through LDS)
-  for (int c = 0; c < C0; ++c) {
-    float f = 0.f;
-    if (p < P) {
-      f = (float)d[(size_t)p * C0 + c];
-      const float gd = w[c] * g0 + w[C0 + c] * g1;
-      dd[(size_t)p * C0 + c] = (__bf16)(f > 0.f ? gd : 0.f);
-    }
-    s[threadIdx.x] = g0 * f;
-    s[256 + threadIdx.x] = g1 * f;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-      if ((int)threadIdx.x < o) {
-        s[threadIdx.x] += s[threadIdx.x + o];
-        s[256 + threadIdx.x] += s[256 + threadIdx.x + o];
-      }
-      __syncthreads();
-    }
-    if (threadIdx.x == 0) {
-      atomicAdd(dW + c, s[0]);
-      atomicAdd(dW + C0 + c, s[256]);
-    }
-    __syncthreads();
+  if (threadIdx.x < 76) {
+    const int h = threadIdx.x / 19, k = threadIdx.x % 19, c = blockIdx.y * 32 + 8 * h;
+    const float v = red[0][h][k] + red[1][h][k] + red[2][h][k] + red[3][h][k];
+    // partial: dW [2][C0], db [2], loss
+    part += (size_t)blockIdx.x * (2 * C0 + 3);
+    if (k < 8) part[c + k] = v;
+    else if (k < 16) part[C0 + c + k - 8] = v;
+    else if (h == 0 && blockIdx.y == 0) part[2 * C0 + (k == 16 ? 2 : k - 17)] = v;
   }
 }
 
@@ -1319,11 +1397,6 @@ __global__ __launch_bounds__(256) void weights_to_bf16_kernel(const float* __res
   const __bf16 h = (__bf16)w[i];
   wf[i] = h;
   if (wt) wt[((size_t)ci * 9 + (8 - t)) * Cout + co] = h;
-}
-
-__global__ void fill_kernel(float* __restrict__ p, long count, float v) {
-  const long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (i < count) p[i] = v;
 }
 
 // ======================================================== host launchers
@@ -1500,14 +1573,23 @@ hipError_t unet_conv3_in(const float2* x, const float* w, const float* b, __bf16
   return hipGetLastError();
 }
 
-hipError_t unet_conv3_in_dw(const float2* x, const __bf16* dY, float* dW, float* db, int n,
-                            int H, int W, int C0, hipStream_t s) {
-  const long P = (long)n * H * W;
-  const int ppb = 2048;
-  const int nk = C0 * 19;  // weights and biases
-  const int threads = std::min(1024, ((nk + 63) / 64) * 64);
-  hipLaunchKernelGGL(conv3_in_dw_kernel, dim3(blocks(P, ppb), (nk + threads - 1) / threads),
-                     dim3(threads), 0, s, x, dY, dW, db, n, H, W, C0, ppb);
+// workgroups of conv3_in_dw_kernel (two per CU, rows dealt round robin)
+static int in_dw_wgs(long rows, int C0) {
+  return (int)std::max(1L, std::min<long>(rows, 2L * device_cus() / (C0 / 32)));
+}
+size_t unet_conv3_in_dw_floats(int n, int H, int C0) {
+  return (size_t)in_dw_wgs((long)n * H, C0) * C0 * 19;
+}
+hipError_t unet_conv3_in_dw(const float2* x, const __bf16* dY, float* dW, float* db, float* ws,
+                            int n, int H, int W, int C0, hipStream_t s) {
+  if (C0 % 32) return hipErrorInvalidValue;
+  const int wgs = in_dw_wgs((long)n * H, C0);
+  hipLaunchKernelGGL(conv3_in_dw_kernel, dim3(wgs, C0 / 32), dim3(512), 0, s, x, dY, ws, n, H, W,
+                     C0);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(partials_kernel, dim3(blocks(C0 * 19, 16)), dim3(256), 0, s, ws, wgs, C0 * 19,
+                     dW, C0 * 18, db, C0, nullptr, 0);
   return hipGetLastError();
 }
 
@@ -1517,11 +1599,24 @@ hipError_t unet_conv1_out(const __bf16* d, const float2* x, const float* w, cons
   return hipGetLastError();
 }
 
+// workgroups of conv1_out_bwd_kernel (eight per CU walk the pixels)
+static int out_bwd_wgs(long P, int C0) {
+  return (int)std::max(1L, std::min<long>((P + 63) / 64, 8L * device_cus() / (C0 / 32)));
+}
+size_t unet_conv1_out_bwd_floats(long P, int C0) {
+  return (size_t)out_bwd_wgs(P, C0) * (2 * C0 + 3);
+}
 hipError_t unet_conv1_out_bwd(const __bf16* d, const float2* out, const float2* u,
                               const float* w, __bf16* dd, float* dW, float* db, float* loss,
-                              long P, int C0, hipStream_t s) {
-  hipLaunchKernelGGL(conv1_out_bwd_kernel, dim3(blocks(P)), dim3(256), 3 * 256 * sizeof(float),
-                     s, d, out, u, w, dd, dW, db, loss, P, C0);
+                              float* ws, long P, int C0, hipStream_t s) {
+  if (C0 % 32) return hipErrorInvalidValue;
+  const int wgs = out_bwd_wgs(P, C0);
+  hipLaunchKernelGGL(conv1_out_bwd_kernel, dim3(wgs, C0 / 32), dim3(256), 0, s, d, out, u, w, dd,
+                     ws, P, C0);
+  const hipError_t e = hipGetLastError();
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL(partials_kernel, dim3(blocks(2 * C0 + 3, 16)), dim3(256), 0, s, ws, wgs,
+                     2 * C0 + 3, dW, 2 * C0, db, 2, loss, 1);
   return hipGetLastError();
 }
 
@@ -1560,12 +1655,6 @@ hipError_t unet_weights_bf16(const float* w, __bf16* wf, __bf16* wt, int Cout, i
                              hipStream_t s) {
   hipLaunchKernelGGL(weights_to_bf16_kernel, dim3(blocks((long)Cout * 9 * Cin)), dim3(256), 0, s,
                      w, wf, wt, Cout, Cin);
-  return hipGetLastError();
-}
-
-hipError_t unet_fill(float* p, long count, float v, hipStream_t s) {
-  if (count <= 0) return hipSuccess;
-  hipLaunchKernelGGL(fill_kernel, dim3(blocks(count)), dim3(256), 0, s, p, count, v);
   return hipGetLastError();
 }
 
