@@ -1311,63 +1311,83 @@ __global__ __launch_bounds__(256) void maxpool2_kernel(const __bf16* __restrict_
 // Gradient into an encoder output e (C channels, H x W) from its two
 // consumers, then through its relu:  g_e = (pool adjoint of gp (H/2 x W/2)
 // routed to the first maximum of each window, row-major) + gskip (channels
-// [0, C) of the decoder's concatenated input gradient, pitch Cs; may be
-// null), times (e > 0).
+// [0, C) of the decoder's concatenated input gradient, pitch Cs), times
+// (e > 0).  One thread per window and 8 channels (16-byte accesses; one
+// channel per thread moved 2 bytes at a time).  Bound by memory.
 __global__ __launch_bounds__(256) void pool_bwd_kernel(const __bf16* __restrict__ e,
                                                        const __bf16* __restrict__ gp,
                                                        const __bf16* __restrict__ gskip, int Cs,
                                                        __bf16* __restrict__ ge, int n, int H,
                                                        int W, int C) {
-  const int H2 = H / 2, W2 = W / 2;
+  const int H2 = H / 2, W2 = W / 2, G = C / 8;
   const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (long)n * H2 * W2 * C) return;
-  const int c = (int)(gid % C);
-  const long q = gid / C;
+  if (gid >= (long)n * H2 * W2 * G) return;
+  const int c = (int)(gid % G) * 8;
+  const long q = gid / G;
   const int x2 = (int)(q % W2), y2 = (int)((q / W2) % H2), img = (int)(q / ((long)W2 * H2));
-  const float g = gp ? (float)gp[q * C + c] : 0.f;
-  float best = -1.f;
-  int arg = 0;
-  size_t idx[4];
+  const bf16x8 g = *(const bf16x8*)(gp + q * C + c);
+  bf16x8 ev[4], gs[4];
+  size_t pix[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
-    const int yy = 2 * y2 + k / 2, xx = 2 * x2 + k % 2;
-    const size_t pix = ((size_t)img * H + yy) * W + xx;
-    idx[k] = pix;
-    const float v = (float)e[pix * C + c];
-    if (k == 0 || v > best) {
-      best = v;
-      arg = k;
+    pix[k] = ((size_t)img * H + 2 * y2 + k / 2) * W + 2 * x2 + k % 2;
+    ev[k] = *(const bf16x8*)(e + pix[k] * C + c);
+    gs[k] = *(const bf16x8*)(gskip + pix[k] * Cs + c);
+  }
+  bf16x8 o[4];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    float best = (float)ev[0][j];
+    int arg = 0;
+#pragma unroll
+    for (int k = 1; k < 4; ++k) {
+      const float v = (float)ev[k][j];
+      if (v > best) {
+        best = v;
+        arg = k;
+      }
+    }
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const float v = (k == arg ? (float)g[j] : 0.f) + (float)gs[k][j];
+      o[k][j] = (__bf16)((float)ev[k][j] > 0.f ? v : 0.f);
     }
   }
 #pragma unroll
-  for (int k = 0; k < 4; ++k) {
-    const size_t pix = idx[k];
-    float v = (k == arg) ? g : 0.f;
-    if (gskip) v += (float)gskip[pix * Cs + c];
-    ge[pix * C + c] = (__bf16)(((float)e[pix * C + c] > 0.f) ? v : 0.f);
-  }
+  for (int k = 0; k < 4; ++k) *(bf16x8*)(ge + pix[k] * C + c) = o[k];
 }
 
 // Adjoint of the nearest x2 upsampling of a decoder input (channels [C1,
 // C1+C) of the concatenated gradient gcat, full resolution, pitch C1 + C),
-// times (a > 0) for the low-resolution activation a (C channels).
+// times (a > 0) for the low-resolution activation a (C channels).  One thread
+// per low-resolution pixel and 8 channels; bound by memory.
 __global__ __launch_bounds__(256) void up_bwd_kernel(const __bf16* __restrict__ gcat, int C1,
                                                      const __bf16* __restrict__ a,
                                                      __bf16* __restrict__ ga, int n, int H2,
                                                      int W2, int C) {
+  const int G = C / 8;
   const long gid = (long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (gid >= (long)n * H2 * W2 * C) return;
-  const int c = (int)(gid % C);
-  const long q = gid / C;
+  if (gid >= (long)n * H2 * W2 * G) return;
+  const int c = (int)(gid % G) * 8;
+  const long q = gid / G;
   const int x2 = (int)(q % W2), y2 = (int)((q / W2) % H2), img = (int)(q / ((long)W2 * H2));
   const int H = 2 * H2, W = 2 * W2, Cc = C1 + C;
-  float s = 0.f;
+  bf16x8 v[4];
 #pragma unroll
   for (int k = 0; k < 4; ++k) {
     const size_t pix = ((size_t)img * H + 2 * y2 + k / 2) * W + 2 * x2 + k % 2;
-    s += (float)gcat[pix * Cc + C1 + c];
+    v[k] = *(const bf16x8*)(gcat + pix * Cc + C1 + c);
   }
-  ga[q * C + c] = (__bf16)(((float)a[q * C + c] > 0.f) ? s : 0.f);
+  const bf16x8 av = *(const bf16x8*)(a + q * C + c);
+  bf16x8 o;
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    float s = 0.f;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) s += (float)v[k][j];
+    o[j] = (__bf16)((float)av[j] > 0.f ? s : 0.f);
+  }
+  *(bf16x8*)(ga + q * C + c) = o;
 }
 
 // Adam on FP32 master weights; refreshes the BF16 copies: Wf [Cout][9][Cin]
@@ -1628,7 +1648,7 @@ hipError_t unet_maxpool2(const __bf16* x, __bf16* y, int n, int H, int W, int C,
 
 hipError_t unet_pool_bwd(const __bf16* e, const __bf16* gp, const __bf16* gskip, int Cs,
                          __bf16* ge, int n, int H, int W, int C, hipStream_t s) {
-  const long work = (long)n * (H / 2) * (W / 2) * C;
+  const long work = (long)n * (H / 2) * (W / 2) * (C / 8);
   hipLaunchKernelGGL(pool_bwd_kernel, dim3(blocks(work)), dim3(256), 0, s, e, gp, gskip, Cs, ge,
                      n, H, W, C);
   return hipGetLastError();
@@ -1636,7 +1656,7 @@ hipError_t unet_pool_bwd(const __bf16* e, const __bf16* gp, const __bf16* gskip,
 
 hipError_t unet_up_bwd(const __bf16* gcat, int C1, const __bf16* a, __bf16* ga, int n, int H2,
                        int W2, int C, hipStream_t s) {
-  const long work = (long)n * H2 * W2 * C;
+  const long work = (long)n * H2 * W2 * (C / 8);
   hipLaunchKernelGGL(up_bwd_kernel, dim3(blocks(work)), dim3(256), 0, s, gcat, C1, a, ga, n, H2,
                      W2, C);
   return hipGetLastError();
