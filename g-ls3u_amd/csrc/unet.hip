@@ -28,8 +28,7 @@ namespace {
 struct Layer {
   int cin = 0, cout = 0, k = 3;       // k: 3 (3x3) or 1 (1x1)
   float *w = nullptr, *b = nullptr;   // FP32 master [cout][k][k][cin], [cout]
-  float *gw = nullptr, *gb = nullptr;
-  float *mw = nullptr, *vw = nullptr, *mb = nullptr, *vb = nullptr;
+  float *gw = nullptr, *gb = nullptr;  // gradients
   __bf16 *wf = nullptr, *wt = nullptr;  // BF16 forward / flipped-transposed copies
   long nw() const { return (long)cout * k * k * cin; }
 };
@@ -48,6 +47,11 @@ struct glsu_unet {
   int levels = 4, base = 32;
   hipStream_t s = nullptr;
   std::vector<Layer> L;  // e0a e0b e1a e1b ... e{L-1}b d{L-2}a d{L-2}b ... d0a d0b out
+  // parameters, gradients and Adam moments of all layers, each flat in the
+  // layers' order (weights, then biases), which is the host's order too: one
+  // copy moves them all and one launch updates them all
+  long count = 0;
+  float *P = nullptr, *G = nullptr, *M = nullptr, *V = nullptr;
   Acts a;
   int step = 0;
   int C(int l) const { return base << l; }
@@ -241,10 +245,32 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
 static void unet_free(glsu_unet* h) {
   if (h->s) hipStreamSynchronize(h->s);
   acts_free(h->a);
+  hipFree(h->P); hipFree(h->G); hipFree(h->M); hipFree(h->V);
   for (auto& l : h->L) {
-    hipFree(l.w); hipFree(l.b); hipFree(l.gw); hipFree(l.gb);
-    hipFree(l.mw); hipFree(l.vw); hipFree(l.mb); hipFree(l.vb);
     hipFree(l.wf); hipFree(l.wt);
+  }
+}
+
+// n draws of N(0, sd^2) by Marsaglia's polar method, the values that
+// std::normal_distribution<double> gives from the same generator; libstdc++'s
+// takes a long double logarithm for every uniform draw where the compiler does
+// not fold it, which made up most of glsu_unet_create (2 M weights: 127 ms
+// against 27 ms)
+static void normal_fill(std::mt19937_64& rng, float* w, long n, double sd) {
+  auto unit = [&] {  // (-1, 1), 53 bits
+    const double u = (double)rng() / 18446744073709551616.0;
+    return 2.0 * (u < 1.0 ? u : std::nextafter(1.0, 0.0)) - 1.0;
+  };
+  for (long i = 0; i < n; i += 2) {
+    double x, y, r2;
+    do {
+      x = unit();
+      y = unit();
+      r2 = x * x + y * y;
+    } while (r2 > 1.0 || r2 == 0.0);
+    const double m = std::sqrt(-2.0 * std::log(r2) / r2);
+    w[i] = (float)(y * m * sd);
+    if (i + 1 < n) w[i + 1] = (float)(x * m * sd);
   }
 }
 
@@ -275,45 +301,40 @@ extern "C" int glsu_unet_create(glsu_unet** out, int levels, int base, unsigned 
     add(h->C(l), h->C(l), 3);
   }
   add(h->C(0), 2, 1);
+  for (auto& l : h->L) h->count += l.nw() + l.cout;
+  const size_t bytes = (size_t)h->count * sizeof(float);
+  bool ok = true;
+  for (float** p : {&h->P, &h->G, &h->M, &h->V}) ok = ok && hipMalloc((void**)p, bytes) == hipSuccess;
+  long at = 0;
+  for (auto& l : h->L) {
+    l.w = h->P + at; l.gw = h->G + at;
+    at += l.nw();
+    l.b = h->P + at; l.gb = h->G + at;
+    at += l.cout;
+    if (ok && l.k == 3 && l.cin % 32 == 0)
+      ok = hipMalloc((void**)&l.wf, l.nw() * 2) == hipSuccess &&
+           hipMalloc((void**)&l.wt, l.nw() * 2) == hipSuccess;
+  }
+  if (!ok) {
+    unet_free(h);
+    delete h;
+    return ufail(GLSU_ERR_DEVICE, "weight allocation failed");
+  }
+  // He-normal weights, zero biases; the output layer starts at zero (identity net)
   std::mt19937_64 rng(seed);
-  for (size_t i = 0; i < h->L.size(); ++i) {
-    Layer& l = h->L[i];
-    const long nw = l.nw();
-    bool ok = hipMalloc((void**)&l.w, nw * 4) == hipSuccess &&
-              hipMalloc((void**)&l.b, l.cout * 4) == hipSuccess &&
-              hipMalloc((void**)&l.gw, nw * 4) == hipSuccess &&
-              hipMalloc((void**)&l.gb, l.cout * 4) == hipSuccess &&
-              hipMalloc((void**)&l.mw, nw * 4) == hipSuccess &&
-              hipMalloc((void**)&l.vw, nw * 4) == hipSuccess &&
-              hipMalloc((void**)&l.mb, l.cout * 4) == hipSuccess &&
-              hipMalloc((void**)&l.vb, l.cout * 4) == hipSuccess;
-    const bool mfma = l.k == 3 && l.cin % 32 == 0;
-    if (ok && mfma)
-      ok = hipMalloc((void**)&l.wf, nw * 2) == hipSuccess &&
-           hipMalloc((void**)&l.wt, nw * 2) == hipSuccess;
-    if (!ok) {
-      unet_free(h);
-      delete h;
-      return ufail(GLSU_ERR_DEVICE, "weight allocation failed");
-    }
-    // He-normal weights, zero biases; the output layer starts at zero (identity net)
-    std::vector<float> w(nw, 0.f), z(l.cout, 0.f);
-    if (i + 1 < h->L.size()) {
-      std::normal_distribution<double> nd(0.0, std::sqrt(2.0 / (l.k * l.k * l.cin)));
-      for (auto& v : w) v = (float)nd(rng);
-    }
-    std::vector<float> zw(nw, 0.f);
-    ok = hipMemcpy(l.w, w.data(), nw * 4, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(l.b, z.data(), l.cout * 4, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(l.mw, zw.data(), nw * 4, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(l.vw, zw.data(), nw * 4, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(l.mb, z.data(), l.cout * 4, hipMemcpyHostToDevice) == hipSuccess &&
-         hipMemcpy(l.vb, z.data(), l.cout * 4, hipMemcpyHostToDevice) == hipSuccess;
-    if (!ok) {
-      unet_free(h);
-      delete h;
-      return ufail(GLSU_ERR_DEVICE, "weight upload failed");
-    }
+  std::vector<float> w(h->count, 0.f);
+  at = 0;
+  for (size_t i = 0; i + 1 < h->L.size(); ++i) {
+    const Layer& l = h->L[i];
+    normal_fill(rng, w.data() + at, l.nw(), std::sqrt(2.0 / (l.k * l.k * l.cin)));
+    at += l.nw() + l.cout;
+  }
+  if (hipMemcpy(h->P, w.data(), bytes, hipMemcpyHostToDevice) != hipSuccess ||
+      hipMemset(h->M, 0, bytes) != hipSuccess || hipMemset(h->V, 0, bytes) != hipSuccess ||
+      hipStreamSynchronize(nullptr) != hipSuccess) {
+    unet_free(h);
+    delete h;
+    return ufail(GLSU_ERR_DEVICE, "weight upload failed");
   }
   if (int rc = refresh_bf16(h)) {
     unet_free(h);
@@ -326,20 +347,14 @@ extern "C" int glsu_unet_create(glsu_unet** out, int levels, int base, unsigned 
 
 extern "C" int glsu_unet_param_count(glsu_unet* h, long* count) {
   if (!h || !count) return ufail(GLSU_ERR_ARG, "null argument");
-  long c = 0;
-  for (auto& l : h->L) c += l.nw() + l.cout;
-  *count = c;
+  *count = h->count;
   return GLSU_OK;
 }
 
 static int copy_params(glsu_unet* h, float* host, bool grads) {
   UTRY(hipStreamSynchronize(h->s));
-  for (auto& l : h->L) {
-    UTRY(hipMemcpy(host, grads ? l.gw : l.w, l.nw() * 4, hipMemcpyDeviceToHost));
-    host += l.nw();
-    UTRY(hipMemcpy(host, grads ? l.gb : l.b, l.cout * 4, hipMemcpyDeviceToHost));
-    host += l.cout;
-  }
+  UTRY(hipMemcpy(host, grads ? h->G : h->P, (size_t)h->count * sizeof(float),
+                 hipMemcpyDeviceToHost));
   return GLSU_OK;
 }
 
@@ -356,12 +371,7 @@ extern "C" int glsu_unet_get_grads(glsu_unet* h, float* host) {
 extern "C" int glsu_unet_set_params(glsu_unet* h, const float* host) {
   if (!h || !host) return ufail(GLSU_ERR_ARG, "null argument");
   UTRY(hipStreamSynchronize(h->s));
-  for (auto& l : h->L) {
-    UTRY(hipMemcpy(l.w, host, l.nw() * 4, hipMemcpyHostToDevice));
-    host += l.nw();
-    UTRY(hipMemcpy(l.b, host, l.cout * 4, hipMemcpyHostToDevice));
-    host += l.cout;
-  }
+  UTRY(hipMemcpy(h->P, host, (size_t)h->count * sizeof(float), hipMemcpyHostToDevice));
   return refresh_bf16(h);
 }
 
@@ -392,10 +402,7 @@ extern "C" int glsu_unet_loss_grad(glsu_unet* h, const void* d_x, const void* d_
 extern "C" int glsu_unet_adam_step(glsu_unet* h, float lr, float beta1, float beta2, float eps) {
   if (!h || !(lr > 0)) return ufail(GLSU_ERR_ARG, "invalid argument");
   ++h->step;
-  for (auto& l : h->L) {
-    UTRY(unet_adam(l.w, l.gw, l.mw, l.vw, l.nw(), lr, beta1, beta2, eps, h->step, h->s));
-    UTRY(unet_adam(l.b, l.gb, l.mb, l.vb, l.cout, lr, beta1, beta2, eps, h->step, h->s));
-  }
+  UTRY(unet_adam(h->P, h->G, h->M, h->V, h->count, lr, beta1, beta2, eps, h->step, h->s));
   return refresh_bf16(h);
 }
 
