@@ -11,6 +11,7 @@
 #include "../../include/glsu.h"
 #include "glsu_internal.h"
 
+#include <algorithm>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -151,7 +152,10 @@ static bool reference_padding_ok(int W, int H, int sx, int sy) {
 static int default_plan(int need, bool t64_only) { return plan_default(need, t64_only); }
 
 // Host-only validation (no device needed): sizes, parameters, padding rule.
-static int validate(int W, int H, const glsu_wff_params* pr, int* planx, int* plany) {
+// ridge: the handle runs the ridge mode, whose column kernel keeps the shortest
+// plan (its per-pixel maximum over all pairs follows the plan's rounding).
+static int validate(int W, int H, const glsu_wff_params* pr, int* planx, int* plany,
+                    bool ridge = false) {
   if (W < 1 || H < 1) return fail(GLSU_ERR_ARG, "invalid size %dx%d", W, H);
   if (!(pr->wxi > 0) || !(pr->wyi > 0) || !(pr->sigma_x > 0) || !(pr->sigma_y > 0) ||
       !(pr->wxh >= pr->wxl) || !(pr->wyh >= pr->wyl))
@@ -162,7 +166,10 @@ static int validate(int W, int H, const glsu_wff_params* pr, int* planx, int* pl
                 "FFT padding is out of range [4096]. Shrink the size of either the image or the "
                 "Gaussian Window!");
   if (*planx < 0) *planx = default_plan(W + sx, true);
-  if (*plany < 0) *plany = default_plan(H + sy, false);
+  if (*plany < 0) {
+    const double nwx = std::floor((pr->wxh - pr->wxl) * (1 / pr->wxi)) + 1;
+    *plany = ridge ? default_plan(H + sy, false) : plan_default_cols(H + sy, nwx * W);
+  }
   if (*planx < 0 || *plany < 0)
     return fail(GLSU_ERR_PADDING, "no compiled FFT length covers %dx%d + half window", W, H);
   bool okx = false, oky = false;
@@ -187,9 +194,10 @@ static int validate_tuning(const glsu_tuning* t) {
   return GLSU_OK;
 }
 
-static int plan_common(WffPlan& p, int W, int H, const glsu_wff_params* pr, const glsu_tuning* t) {
+static int plan_common(WffPlan& p, int W, int H, const glsu_wff_params* pr, const glsu_tuning* t,
+                       bool ridge = false) {
   int planx = t ? t->planx : -1, plany = t ? t->plany : -1;
-  if (int rc = validate(W, H, pr, &planx, &plany)) return rc;
+  if (int rc = validate(W, H, pr, &planx, &plany, ridge)) return rc;
   std::string err;
   int rc = wff_plan_init(p, W, H, pr->sigma_x, pr->wxl, pr->wxh, pr->wxi, pr->sigma_y, pr->wyl,
                          pr->wyh, pr->wyi, pr->thr, planx, plany, t ? t->cols_waves : -1,
@@ -274,7 +282,7 @@ extern "C" int glsu_wft2_create_tuned(glsu_wft2** out, int W, int H, int type,
   if (type != GLSU_WFF && type != GLSU_WFR) return fail(GLSU_ERR_ARG, "unknown WFT type %d", type);
   {
     int px = t ? t->planx : -1, py = t ? t->plany : -1;
-    if (int rc = validate(W, H, pr, &px, &py)) return rc;
+    if (int rc = validate(W, H, pr, &px, &py, type == GLSU_WFR)) return rc;
     if (int rc = validate_tuning(t)) return rc;
     if (type == GLSU_WFR)
       if (int rc = validate_wfr(W, H, pr)) return rc;
@@ -282,7 +290,7 @@ extern "C" int glsu_wft2_create_tuned(glsu_wft2** out, int W, int H, int type,
   if (int rc = check_device()) return rc;
   auto* h = new glsu_wft2();
   h->type = type;
-  int rc = plan_common(h->p, W, H, pr, t);
+  int rc = plan_common(h->p, W, H, pr, t, type == GLSU_WFR);
   if (rc) { delete h; return rc; }
   if (type == GLSU_WFR && (rc = wfr_alloc(h->p, h->wfr)) != GLSU_OK) {
     wfr_free(h->wfr);
@@ -1138,6 +1146,14 @@ extern "C" int glsu_dpra_batch_create(glsu_dpra_batch** out, const glsu_seq_desc
     int first = -1;
     for (int i = 0; i < n; ++i)
       if (cls_of[i] == (int)c && first < 0) first = i;
+    if (keys[c].rw < 0) {  // the class's rows share its launches
+      int rows = 0, E = 0;
+      for (int i = 0; i < n; ++i)
+        if (cls_of[i] == (int)c) rows += seqs[i].height;
+      for (const FftPlanInfo& q : fft_plans())
+        if (q.id == keys[c].px) E = q.E;
+      keys[c].rw = rows_waves_default(E, rows);
+    }
     std::string err;
     int rc = wff_plan_init(bc.p, seqs[first].width, seqs[first].height, pr->sigma_x, pr->wxl,
                            pr->wxh, pr->wxi, pr->sigma_y, pr->wyl, pr->wyh, pr->wyi, pr->thr,

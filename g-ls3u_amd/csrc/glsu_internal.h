@@ -31,7 +31,7 @@ struct WffPlan {
   int planx = -1, plany = -1;  // FFT plan ids along x (rows) and y (columns)
   int Nx = 0, Ny = 0;
   int cols_waves = 4, rows_waves = 1;  // launch shapes
-  int ls_tile = 1;                      // DPRA least-squares tile shape (launch_dpra_ls)
+  int ls_tile = 3;                      // DPRA least-squares tile shape (launch_dpra_ls)
   // device buffers
   // window spectra / N, lane-major: [w][j][lane] = bin kbase(lane) + koff(j).
   // Real: the window is even, so its modulated spectrum has no imaginary part.
@@ -90,6 +90,11 @@ void wff_plan_free(WffPlan& p);
 int wff_plan_geometry(WffPlan& p, int W, int H, double sigx, double wxl, double wxh, double wxi,
                       double sigy, double wyl, double wyh, double wyi, double thr, int planx,
                       int plany, int cols_waves, int rows_waves, const char** err);
+// Default column plan of the filter for `items` columns over all planes.
+int plan_default_cols(int need, double items);
+// Default waves per row of the row kernels for `rows` rows in one launch and a
+// plan of E points per lane.
+int rows_waves_default(int E, int rows);
 // Default plan for a padded length >= need (row plans: t64_only).
 int plan_default(int need, bool t64_only);
 // wff_plan_init's tables (windows, spectra, twiddles; the threshold when

@@ -80,7 +80,8 @@ extern "C" int glsu_wft2_compute_noalloc(int width, int height, const glsu_wff_p
   // the reference constructor's padding rule (WFT/WFT2_CPU.cpp:710-724)
   if (W + 2 * sx > 4096 || H + 2 * sy > 4096)
     return fail_noalloc(GLSU_ERR_PADDING, "FFT padding is out of range [4096]");
-  const int planx = plan_default(W + sx, true), plany = plan_default(H + sy, false);
+  const double nwx = std::floor((pr->wxh - pr->wxl) * (1 / pr->wxi)) + 1;
+  const int planx = plan_default(W + sx, true), plany = plan_default_cols(H + sy, nwx * W);
   if (planx < 0 || plany < 0)
     return fail_noalloc(GLSU_ERR_PADDING, "no compiled FFT length covers the size + half window");
   WffPlan p;

@@ -141,6 +141,24 @@ int plan_default(int need, bool t64_only) {
   return (plan_row(first)->N < 0.8 * plan_row(best64)->N) ? first : best64;
 }
 
+// Column plans of the filter for `items` columns (planes x width): a narrow plan
+// packs several transforms into a wavefront, which pays once the launch has
+// four wavefronts' worth of columns per SIMD; below that it leaves SIMDs empty
+// and every column's chain takes longer on fewer lanes.  Measured, 16 lanes
+// (320 points) against 64 lanes (512 points), 256 rows, 5 planes: 96 columns
+// 28.7 / 16.4 us, 256 29.8 / 19.8, 600 32.4 / 26.9, 900 38.5 / 35.9, 1400 41.5
+// / 46.5; 192 against 256 points, 130 rows: 256 18.8 / 13.7, 900 23.4 / 21.5,
+// 1400 25.7 / 28.6.  The 32-lane plans were slower at every width.
+int plan_default_cols(int need, double items) {
+  const int best64 = smallest_plan(need, true);
+  if (best64 >= 0 && items < 4096) return best64;
+  int narrow = -1;
+  for (const PlanRow& r : kPlanRows)
+    if (r.T == 16 && r.N >= need && (narrow < 0 || r.N < plan_row(narrow)->N)) narrow = r.id;
+  if (narrow < 0) return best64 >= 0 ? best64 : smallest_plan(need, false);
+  return best64 < 0 || plan_row(narrow)->N < 0.8 * plan_row(best64)->N ? narrow : best64;
+}
+
 // Window spectra in the order the kernels read them: entry (r, j, lane) holds
 // spectral bin kbase(lane) + koff(j) of row r, so that register j of every
 // lane of a transform is one contiguous T-element run (a coalesced load).
@@ -296,6 +314,20 @@ static hipError_t upload(V*& dptr, const std::vector<V>& h) {
   return hipMemcpy(dptr, h.data(), sizeof(V) * h.size(), hipMemcpyHostToDevice);
 }
 
+// Waves per row of the row kernels.  Two waves per SIMD (2048 on the chip) fit
+// up to 20 points per lane; a launch of fewer rows leaves SIMDs empty while
+// every row walks its wx one after the other, so the rows are split over
+// waves as long as all of them are resident at once.  Measured, 1 / 2 / 4
+// waves, forward + inverse row kernels of three frames: 256 rows 66 / 58 / 55
+// us, 512 rows 104 / 92 / 89, 768 rows 133 / 120 / 138, 1024 rows 176 / 154 /
+// 194; with 24 points per lane (900 rows) 265 / 330 / 452.
+int rows_waves_default(int E, int rows) {
+  if (E > 20) return 1;
+  int w = 1;
+  while (2 * w <= kRowWavesMax && 2 * w * rows <= 2048) w *= 2;
+  return w;
+}
+
 int wff_plan_geometry(WffPlan& p, int W, int H, double sigx, double wxl, double wxh, double wxi,
                       double sigy, double wyl, double wyh, double wyi, double thr, int planx,
                       int plany, int cols_waves, int rows_waves, const char** err) {
@@ -334,9 +366,14 @@ int wff_plan_geometry(WffPlan& p, int W, int H, double sigx, double wxl, double 
   p.planx = planx; p.plany = plany;
   p.Nx = px->N; p.Ny = py->N;
   // rows: one wavefront per transform, up to kRowWavesMax waves per row
-  p.rows_waves = 1;
-  if (rows_waves >= 1 && rows_waves <= kRowWavesMax) p.rows_waves = std::min(rows_waves, p.nwx);
+  if (rows_waves < 1 || rows_waves > kRowWavesMax) rows_waves = rows_waves_default(px->E, H);
+  p.rows_waves = std::min(rows_waves, p.nwx);
+  // columns: workgroups of four waves share one twiddle table best; a launch of
+  // few columns spreads more evenly over the CUs in pairs (256 x 256, 5 planes:
+  // 19.8 / 18.4 us with 4 / 2; 371 x 366, 7 planes 28.2 / 27.1; 1024 x 1024, 5
+  // planes 121 / 127)
   if (cols_waves == 1 || cols_waves == 2 || cols_waves == 4) p.cols_waves = cols_waves;
+  else if ((double)p.nwx * W * py->T < 3072 * 64) p.cols_waves = 2;
   // keep dynamic LDS per workgroup within 64 KiB
   while (p.cols_waves > 1 && plan_smem_bytes(plany, p.cols_waves, true) > 65536) p.cols_waves /= 2;
   while (p.rows_waves > 1 && plan_smem_bytes(planx, p.rows_waves) > 65536) --p.rows_waves;
@@ -362,7 +399,12 @@ int wff_plan_init(WffPlan& p, int W, int H, double sigx, double wxl, double wxh,
     auto t = window_spectrum(gx, p.sx, wxl + (double)k * wxi, p.Nx);
     hx.insert(hx.end(), t.begin(), t.end());
   }
-  for (int k = 0; k < p.nwy; ++k) {
+  // the same window, grid and length on both axes share one table (each entry
+  // is a sum of 2 s + 1 cosines: 1 ms of host time at 512 points, 5 rows)
+  const bool same = p.Nx == p.Ny && p.sx == p.sy && p.nwx == p.nwy && sigx == sigy &&
+                    wxl == wyl && wxi == wyi;
+  if (same) hy = hx;
+  for (int k = same ? p.nwy : 0; k < p.nwy; ++k) {
     auto t = window_spectrum(gy, p.sy, wyl + (double)k * wyi, p.Ny);
     hy.insert(hy.end(), t.begin(), t.end());
   }

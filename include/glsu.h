@@ -54,9 +54,10 @@ typedef struct glsu_wff_params {
  * FFT plan ids (glsu_fft_plans) along rows and columns; cols_waves:
  * wavefronts per workgroup of the column kernel (1, 2 or 4); rows_waves:
  * wavefronts per row of the row kernels (1..4); ls_tile: pixel tile of the
- * DPRA least-squares kernel, 1 = 64x8 (default), 2 = 64x4, 3 = 32x8,
+ * DPRA least-squares kernel, 1 = 64x8, 2 = 64x4, 3 = 32x8 (default),
  * 4 = 128x4, 5 = 64x16, 6 = 32x16 (batches always use 64x8).  Results do not
- * depend on the FFT plans beyond FP32 rounding and not at all on the launch
+ * depend on the FFT plans and rows_waves (the order of the sum over wx) beyond
+ * FP32 rounding and not at all on the other launch
  * shapes.  No reference counterpart (the reference fixes its DPRA blocks,
  * DPRA/dpra_cudaf.cu:121-122). */
 typedef struct glsu_tuning {

@@ -142,3 +142,30 @@ def test_every_fft_plan_matches_oracle(oracle):
         rel = np.abs(out - ref).max() / np.abs(ref).max()
         say(f"   rel={rel:.2e}")
         assert rel < 1e-4, p
+
+
+@pytest.mark.parametrize("W,H,T", [
+    (818, 130, 64),   # 5 planes x 818 = 4090 columns: one transform per wavefront
+    (820, 130, 16),   # 4100 columns: four narrow transforms per wavefront (192 points)
+    (1000, 226, 64),  # exactly 256 points: no narrow plan is shorter
+    (1000, 227, 16),  # one more: 320 narrow against 512
+    (820, 290, 16),   # exactly 320 points
+    (820, 291, 64),   # one more: 512 points, no narrow plan
+    (33, 40, 64),     # a small image: rows over four wavefronts, columns in pairs
+])
+def test_default_column_plans_at_their_limits_match_oracle(oracle, W, H, T):
+    """The default column plan follows the number of columns (planes x width)
+    and the padded length; both sides of each limit against the oracle."""
+    rng = np.random.default_rng(W + H)
+    ph = 0.05 * np.arange(W)[None, :] - 0.08 * np.arange(H)[:, None] + rng.normal(0, 0.4, (H, W))
+    f = np.exp(1j * ph).astype(np.complex64)
+    ref = oracle.WFF2(W, H, 10.0, -0.2, 0.2, 0.1)(f.astype(np.complex128))
+    w = glsu.WFT2(W, H, params=glsu.wff_params(10.0, -0.2, 0.2, 0.1))
+    plans = {p["id"]: p for p in glsu.fft_plans()}
+    assert plans[w.tuning()["plany"]]["T"] == T, w.tuning()
+    out = w(torch.from_numpy(f).cuda()).cpu().numpy()
+    rel = np.abs(out - ref).max() / np.abs(ref).max()
+    rms, _ = wrapped_err(np.angle(out), np.angle(ref))
+    say(f"   {W}x{H} {w.tuning()} rel={rel:.2e} phase rms={rms:.2e}")
+    assert rel < 1e-4
+    assert rms < 1e-4
