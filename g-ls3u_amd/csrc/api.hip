@@ -1033,7 +1033,22 @@ struct glsu_dpra_batch {
   int* h_frame = nullptr;       // pinned
   int ntiles = 0, grid_ls = 0;
   std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // by frame dtype
+  std::map<int, bool> seen;  // frame dtypes of earlier calls
   hipEvent_t e0 = nullptr, e1 = nullptr;
+  // Side streams: the classes' WFF2 chains are independent between the
+  // threshold and the frame's end.  Where no class gives the column kernel more
+  // than four rounds of resident workgroups, its launches leave much of the chip
+  // idle at their ends (and never fill it where there is less than one round),
+  // so the classes are dealt over up to four streams (the hardware queues of a
+  // process) and run side by side: five images of 0.07 to 0.8 Mpx take 282 us a
+  // frame against 427 one class after the other.  Classes of many rounds fill
+  // the chip by themselves and lose locality side by side (64 images up to
+  // 2048 x 2048: 2.91 k frames/s against 3.21 k), so they stay on one stream.
+  static constexpr int kSide = 3;
+  int ns = 0;              // side streams in use
+  std::vector<int> order;  // classes by falling work
+  hipStream_t side[kSide] = {};
+  hipEvent_t fork = nullptr, join[kSide] = {};
 };
 
 static void batch_free(glsu_dpra_batch* h) {
@@ -1054,6 +1069,11 @@ static void batch_free(glsu_dpra_batch* h) {
   if (h->h_frame) hipHostFree(h->h_frame);
   if (h->e0) hipEventDestroy(h->e0);
   if (h->e1) hipEventDestroy(h->e1);
+  for (int k = 0; k < glsu_dpra_batch::kSide; ++k) {
+    if (h->side[k]) hipStreamSynchronize(h->side[k]), hipStreamDestroy(h->side[k]);
+    if (h->join[k]) hipEventDestroy(h->join[k]);
+  }
+  if (h->fork) hipEventDestroy(h->fork);
   if (h->own && h->s) hipStreamDestroy(h->s);
   if (h->cap) hipStreamDestroy(h->cap);
 }
@@ -1215,6 +1235,20 @@ extern "C" int glsu_dpra_batch_create(glsu_dpra_batch** out, const glsu_seq_desc
   if (h->grid_ls < 1) return bail(fail(GLSU_ERR_DEVICE, "occupancy query failed"));
   hipEventCreate(&h->e0);
   hipEventCreate(&h->e1);
+  for (size_t c = 0; c < h->cls.size(); ++c) h->order.push_back((int)c);
+  auto work = [&](int c) { return (double)h->cls[c].p.Ny * h->cls[c].bc.ncolblk; };
+  std::stable_sort(h->order.begin(), h->order.end(),
+                   [&](int a, int b) { return work(a) > work(b); });
+  bool small = true;
+  for (auto& c : h->cls) small = small && c.bc.ncolblk <= 4 * c.bc.grid_cols;
+  const int ns = small ? std::min((int)h->cls.size() - 1, (int)glsu_dpra_batch::kSide) : 0;
+  h->ns = ns;
+  if (ns > 0 && hipEventCreateWithFlags(&h->fork, hipEventDisableTiming) != hipSuccess)
+    return bail(fail(GLSU_ERR_DEVICE, "event creation failed"));
+  for (int k = 0; k < ns; ++k)
+    if (hipStreamCreateWithFlags(&h->side[k], hipStreamNonBlocking) != hipSuccess ||
+        hipEventCreateWithFlags(&h->join[k], hipEventDisableTiming) != hipSuccess)
+      return bail(fail(GLSU_ERR_DEVICE, "stream creation failed"));
   *out = h;
   return GLSU_OK;
 }
@@ -1225,9 +1259,33 @@ static int batch_step(glsu_dpra_batch* h, int dtype, hipStream_t st) {
   HIP_TRY(launch_dpra_ls_batch(h->d_tab, (int)h->img.size(), h->ntiles, h->grid_ls, dtype,
                                h->d_frame, st));
   HIP_TRY(launch_thr_batch(h->d_tab, (int)h->img.size(), st));
-  for (auto& c : h->cls) HIP_TRY(launch_rows_fwd_batch(c.bc, st));
-  for (auto& c : h->cls) HIP_TRY(launch_cols_batch(c.bc, st));
-  for (auto& c : h->cls) HIP_TRY(launch_rows_inv_batch(c.bc, h->d_frame, st));
+  const int ns = h->ns;
+  if (ns == 0) {
+    for (auto& c : h->cls) HIP_TRY(launch_rows_fwd_batch(c.bc, st));
+    for (auto& c : h->cls) HIP_TRY(launch_cols_batch(c.bc, st));
+    for (auto& c : h->cls) HIP_TRY(launch_rows_inv_batch(c.bc, h->d_frame, st));
+    HIP_TRY(launch_frame_advance(h->d_frame, st));
+    return GLSU_OK;
+  }
+  // the largest class stays on st, the others go round the side streams
+  HIP_TRY(hipEventRecord(h->fork, st));
+  for (int k = 0; k < ns; ++k) HIP_TRY(hipStreamWaitEvent(h->side[k], h->fork, 0));
+  hipError_t le = hipSuccess;
+  for (size_t i = 0; i < h->order.size() && le == hipSuccess; ++i) {
+    const BatchClass& bc = h->cls[h->order[i]].bc;
+    const int k = (int)(i % (size_t)(ns + 1)) - 1;
+    hipStream_t cs = k < 0 ? st : h->side[k];
+    le = launch_rows_fwd_batch(bc, cs);
+    if (le == hipSuccess) le = launch_cols_batch(bc, cs);
+    if (le == hipSuccess) le = launch_rows_inv_batch(bc, h->d_frame, cs);
+  }
+  // the side streams join st also after a failed launch: a capture has to end
+  // with every forked stream joined
+  for (int k = 0; k < ns; ++k) {
+    HIP_TRY(hipEventRecord(h->join[k], h->side[k]));
+    HIP_TRY(hipStreamWaitEvent(st, h->join[k], 0));
+  }
+  HIP_TRY(le);
   HIP_TRY(launch_frame_advance(h->d_frame, st));
   return GLSU_OK;
 }
@@ -1259,6 +1317,12 @@ extern "C" int glsu_dpra_batch_run(glsu_dpra_batch* h, const void* const* frames
                          hipMemcpyHostToDevice, h->s));
   HIP_TRY(hipMemcpyAsync(h->d_frame, h->h_frame, sizeof(int), hipMemcpyHostToDevice, h->s));
   if (ms) HIP_TRY(hipEventRecord(h->e0, h->s));
+  // the first call of a few frames launches them directly: capturing and
+  // instantiating the graph (about 0.3 ms) costs more than replaying it saves
+  // there (13 us a frame)
+  bool& seen = h->seen[dtype];
+  if (use_graph && !seen && nframes < 16) use_graph = 0;
+  seen = true;
   if (use_graph) {
     auto it = h->graphs.find(dtype);
     if (it == h->graphs.end()) {
