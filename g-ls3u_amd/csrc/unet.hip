@@ -16,6 +16,7 @@
 #include <cstdio>
 #include <random>
 #include <string>
+#include <utility>
 #include <vector>
 
 namespace glsu {
@@ -81,42 +82,40 @@ static void acts_free(Acts& a) {
   a = Acts{};
 }
 
+// One device allocation for several buffers: each (pointer, bytes) at a
+// 256-byte boundary.
+static int arena_alloc(Acts& a, const std::vector<std::pair<void**, size_t>>& want) {
+  size_t total = 0;
+  for (auto& w : want) total += (w.second + 255) & ~(size_t)255;
+  char* p = nullptr;
+  if (hipMalloc((void**)&p, total) != hipSuccess)
+    return ufail(GLSU_ERR_DEVICE, "activation allocation failed");
+  a.bufs.push_back(p);
+  for (auto& w : want) {
+    *w.first = p;
+    p += (w.second + 255) & ~(size_t)255;
+  }
+  return GLSU_OK;
+}
+
+// the forward pass's activations
 static int acts_alloc(glsu_unet* h, int n, int H, int W) {
   Acts& a = h->a;
   if (a.n == n && a.H == H && a.W == W) return GLSU_OK;
   acts_free(a);
-  a.n = n; a.H = H; a.W = W;
-  auto get = [&](size_t elems, size_t sz) -> void* {
-    void* p = nullptr;
-    if (hipMalloc(&p, elems * sz) != hipSuccess) return nullptr;
-    a.bufs.push_back(p);
-    return p;
-  };
-  const int Lv = h->levels;
-  for (int l = 0; l < Lv; ++l) {
-    const size_t px = (size_t)n * (H >> l) * (W >> l), c = h->C(l);
-    a.ea[l] = (__bf16*)get(px * c, 2);
-    a.e[l] = (__bf16*)get(px * c, 2);
-    a.ge[l] = (__bf16*)get(px * c, 2);
-    a.gea[l] = (__bf16*)get(px * c, 2);
-    if (l < Lv - 1) {
-      const size_t pxl = px / 4;
-      a.p[l] = (__bf16*)get(pxl * c, 2);
-      a.gp[l] = (__bf16*)get(pxl * c, 2);
-      a.da[l] = (__bf16*)get(px * c, 2);
-      a.d[l] = (__bf16*)get(px * c, 2);
-      a.gd[l] = (__bf16*)get(px * c, 2);
-      a.gda[l] = (__bf16*)get(px * c, 2);
-      a.gcat[l] = (__bf16*)get(px * (c + h->C(l + 1)), 2);
-      if (!a.p[l] || !a.gp[l] || !a.da[l] || !a.d[l] || !a.gd[l] || !a.gda[l] || !a.gcat[l])
-        return ufail(GLSU_ERR_DEVICE, "activation allocation failed");
+  std::vector<std::pair<void**, size_t>> want;
+  for (int l = 0; l < h->levels; ++l) {
+    const size_t b = (size_t)n * (H >> l) * (W >> l) * h->C(l) * sizeof(__bf16);
+    want.push_back({(void**)&a.ea[l], b});
+    want.push_back({(void**)&a.e[l], b});
+    if (l < h->levels - 1) {
+      want.push_back({(void**)&a.p[l], b / 4});
+      want.push_back({(void**)&a.da[l], b});
+      want.push_back({(void**)&a.d[l], b});
     }
-    if (!a.ea[l] || !a.e[l] || !a.ge[l] || !a.gea[l])
-      return ufail(GLSU_ERR_DEVICE, "activation allocation failed");
   }
-  a.out = (float2*)get((size_t)n * H * W, sizeof(float2));
-  a.loss = (float*)get(1, sizeof(float));
-  if (!a.out || !a.loss) return ufail(GLSU_ERR_DEVICE, "activation allocation failed");
+  if (int rc = arena_alloc(a, want)) return rc;
+  a.n = n; a.H = H; a.W = W;
   return GLSU_OK;
 }
 
@@ -169,24 +168,35 @@ static int forward(glsu_unet* h, const float2* x, float2* out, int n, int H, int
   return GLSU_OK;
 }
 
-// scratch of the weight gradients: the largest layer's partial sums
-static int grad_ws_alloc(glsu_unet* h, int n, int H, int W) {
+// the backward pass's buffers (a network that is only run never has them):
+// activation gradients, the output, the loss, and scratch for the largest
+// layer's partial sums
+static int grads_alloc(glsu_unet* h, int n, int H, int W) {
   Acts& a = h->a;
   if (a.ws) return GLSU_OK;
+  std::vector<std::pair<void**, size_t>> want;
+  const size_t P = (size_t)n * H * W;
   size_t m = std::max(unet_conv3_in_dw_floats(n, H, h->C(0)),
-                      unet_conv1_out_bwd_floats((long)n * H * W, h->C(0)));
+                      unet_conv1_out_bwd_floats((long)P, h->C(0)));
   for (int l = 0; l < h->levels; ++l) {
     const int Hl = H >> l, Wl = W >> l, C = h->C(l);
+    const size_t px = (size_t)n * Hl * Wl, b = px * C * sizeof(__bf16);
+    want.push_back({(void**)&a.ge[l], b});
+    want.push_back({(void**)&a.gea[l], b});
     m = std::max(m, unet_conv3_dw_floats(C, C, 0, n, Hl, Wl));
     if (l > 0) m = std::max(m, unet_conv3_dw_floats(C, h->C(l - 1), 0, n, Hl, Wl));
-    if (l + 1 < h->levels) m = std::max(m, unet_conv3_dw_floats(C, C, h->C(l + 1), n, Hl, Wl));
+    if (l < h->levels - 1) {
+      want.push_back({(void**)&a.gp[l], b / 4});
+      want.push_back({(void**)&a.gd[l], b});
+      want.push_back({(void**)&a.gda[l], b});
+      want.push_back({(void**)&a.gcat[l], px * (C + h->C(l + 1)) * sizeof(__bf16)});
+      m = std::max(m, unet_conv3_dw_floats(C, C, h->C(l + 1), n, Hl, Wl));
+    }
   }
-  void* p = nullptr;
-  if (hipMalloc(&p, m * sizeof(float)) != hipSuccess)
-    return ufail(GLSU_ERR_DEVICE, "gradient scratch allocation failed");
-  a.bufs.push_back(p);
-  a.ws = (float*)p;
-  return GLSU_OK;
+  want.push_back({(void**)&a.out, P * sizeof(float2)});
+  want.push_back({(void**)&a.loss, sizeof(float)});
+  want.push_back({(void**)&a.ws, m * sizeof(float)});
+  return arena_alloc(a, want);
 }
 
 // loss and gradients for targets u
@@ -194,7 +204,6 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
   Acts& a = h->a;
   const int Lv = h->levels;
   hipStream_t s = h->s;
-  if (int rc = grad_ws_alloc(h, n, H, W)) return rc;
   const long P = (long)n * H * W;
   Layer& o = h->out();
   UTRY(unet_conv1_out_bwd(a.d[0], a.out, u, o.w, a.gd[0], o.gw, o.gb, a.loss, a.ws, P,
@@ -388,6 +397,7 @@ extern "C" int glsu_unet_loss_grad(glsu_unet* h, const void* d_x, const void* d_
   if (!h || !d_x || !d_u) return ufail(GLSU_ERR_ARG, "null argument");
   if (int rc = check_shape(h, n, H, W)) return rc;
   if (int rc = acts_alloc(h, n, H, W)) return rc;
+  if (int rc = grads_alloc(h, n, H, W)) return rc;
   if (int rc = forward(h, (const float2*)d_x, h->a.out, n, H, W)) return rc;
   if (int rc = backward(h, (const float2*)d_x, (const float2*)d_u, n, H, W)) return rc;
   if (loss) {
