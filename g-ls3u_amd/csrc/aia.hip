@@ -26,15 +26,18 @@
 // writes the next weights.  (A last-block-done reduction inside the pass would
 // need an agent-scope release/acquire per block, which on this multi-XCD part
 // writes back and invalidates the XCD's L2 -- evicting the frames the other
-// blocks are reading.)  A device flag makes the remaining launches exit at
-// once after convergence, so iterations need no host round trip; results are
-// bitwise reproducible run to run.
+// blocks are reading.)  Each solve stores the number of completed iterations and
+// whether the loop is over into pinned host memory; the host enqueues two
+// iterations ahead of that count and stops when it is over, and a device flag
+// makes the one launched too many exit at once.  Results are bitwise
+// reproducible run to run.
 //
 // Frames with more than 32 images are processed in chunks of 32 frames per
 // block group (each group recomputes the phase of its pixels and accumulates
 // the shift sums of its own frames).
 #include <hip/hip_runtime.h>
 
+#include <chrono>
 #include <cmath>
 #include <cstdarg>
 #include <cstdint>
@@ -55,7 +58,12 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kSolveThreads = 1024;  // the one-block shift-step solve
 constexpr int kMaxFrames = 1024;
-constexpr int kLaunchGroup = 16;  // iterations enqueued between convergence polls
+// Iterations enqueued ahead of the last one known to be complete: the next is
+// launched while one runs, so the stream does not drain, and at most one
+// iteration is enqueued in vain (each idle launch takes 5-10 us of stream time;
+// groups of sixteen cost a 371 x 366 run of six iterations more than the
+// iterations themselves, 369 us in all).
+constexpr int kLead = 2;
 
 struct AiaCtl {
   int done;      // 1 once converged, out of iterations, or failed
@@ -266,13 +274,17 @@ __device__ __forceinline__ void phase_group(const T* __restrict__ f, int kb, int
 // ---- kernels ------------------------------------------------------------------
 // Per-frame intensity sums sum_j I_k(j) (constant over the iterations): block
 // (b, k) sums quads b*256 + tid (stride Gs*256) of frame k in FP64.  Block
-// (0, 0) also initialises the control block (the shifts and the first
-// weights come from the host).
+// (0, 0) also initialises the control block and fetches the shifts and the
+// first weights from the host's pinned image (a copy on the stream would be one
+// more launch).
 template <typename T>
 __global__ __launch_bounds__(kThreads) void aia_frame_sums_kernel(
     const T* __restrict__ f, long long N, int vec, double* __restrict__ part,
-    AiaCtl* __restrict__ ctl, int max_iter, double max_err, int timing) {
+    AiaCtl* __restrict__ ctl, int max_iter, double max_err, int timing,
+    const uint32_t* __restrict__ h_state, uint32_t* __restrict__ state, int words) {
   const int k = blockIdx.y, Gs = gridDim.x;
+  if (blockIdx.x == 0 && k == 0)
+    for (int i = threadIdx.x; i < words; i += kThreads) state[i] = h_state[i];
   if (blockIdx.x == 0 && k == 0 && threadIdx.x == 0) {
     const double err = max_err * 2.0;
     ctl->iters = 0;
@@ -453,6 +465,13 @@ __global__ __launch_bounds__(kThreads) void aia_pass_kernel(
   }
 }
 
+// Tells the host how far the loop is: one word, so that it is never seen half
+// written; nothing else is read on the strength of it.
+__device__ __forceinline__ void report(unsigned long long* progress, int done, int iters) {
+  __hip_atomic_store(progress, (unsigned long long)done << 32 | (unsigned)iters, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Shift step of one iteration (one block): reduces the pass's partials in a
 // fixed order, solves the M shift systems in FP64, tests convergence, and
 // writes the next phase-step weights and the control block.  After the done
@@ -463,7 +482,8 @@ __global__ __launch_bounds__(kSolveThreads) void aia_solve_kernel(
     int M, long long N, int G, int Gtot, AiaCtl* __restrict__ ctl, float* __restrict__ w1g,
     float* __restrict__ w2g, double* __restrict__ delta, double* __restrict__ Tk,
     const float* __restrict__ part, const double* __restrict__ sums_part, int Gs_first,
-    int max_iter, double max_err, int err_mode, int timing) {
+    int max_iter, double max_err, int err_mode, int timing,
+    unsigned long long* __restrict__ progress) {
   constexpr int kWaves = kSolveThreads / 64;
   extern __shared__ unsigned char smem_raw[];
   double* tot = reinterpret_cast<double*>(smem_raw);  // [5 + 2M]: five sums, then P_k, Q_k
@@ -540,6 +560,7 @@ __global__ __launch_bounds__(kSolveThreads) void aia_solve_kernel(
     if (tid == 0) {
       ctl->status = 20 + s_info;
       ctl->done = 1;
+      report(progress, 1, s_iters);
     }
     return;
   }
@@ -585,7 +606,10 @@ __global__ __launch_bounds__(kSolveThreads) void aia_solve_kernel(
     ctl->iters = it;
     ctl->err = m;
     ctl->status = s_info ? 10 + s_info : 0;
-    ctl->done = (s_info != 0) || (timing ? it >= max_iter : !(m > max_err && it < max_iter));
+    const int done =
+        (s_info != 0) || (timing ? it >= max_iter : !(m > max_err && it < max_iter));
+    ctl->done = done;
+    report(progress, done, it);
   }
   __syncthreads();
   for (int k = tid; k < M; k += kSolveThreads) {
@@ -606,11 +630,13 @@ template <typename T, int GS>
 __global__ __launch_bounds__(kThreads) void aia_final_kernel(
     const T* __restrict__ f, int M, long long N, int vec, const AiaCtl* __restrict__ ctl,
     const float* __restrict__ w1g, const float* __restrict__ w2g,
-    const double* __restrict__ delta, float* __restrict__ phi, float* __restrict__ dout) {
+    const double* __restrict__ delta, float* __restrict__ phi, AiaCtl* __restrict__ h_ctl,
+    float* __restrict__ h_dout) {
   extern __shared__ unsigned char smem_raw[];
   float* sw1 = reinterpret_cast<float*>(smem_raw);
   const int Mp = padded_frames(M);
   float* sw2 = sw1 + Mp;
+  if (blockIdx.x == 0 && threadIdx.x == 0) *h_ctl = *ctl;  // pinned host memory
   if (ctl->status) return;
   for (int k = threadIdx.x; k < Mp; k += kThreads) {
     sw1[k] = k < M ? w1g[k] : 0.f;
@@ -621,7 +647,7 @@ __global__ __launch_bounds__(kThreads) void aia_final_kernel(
     for (int k = threadIdx.x; k < M; k += kThreads) {
       double s, c;
       sincos(delta[k] - d0, &s, &c);
-      dout[k] = (float)atan2(s, c);
+      h_dout[k] = (float)atan2(s, c);
     }
   __syncthreads();
   const long long nq = (N + 3) >> 2;
@@ -649,8 +675,7 @@ __global__ __launch_bounds__(kThreads) void aia_final_kernel(
 // ---- handle -------------------------------------------------------------------
 // Device memory (one allocation): control block; shifts (FP64) and phase-step
 // weights (FP32, padded to a multiple of 32) contiguous, so one copy sets all
-// three from the host; frame sums; pass partials; frame-sum partials; output
-// shifts.
+// three from the host; frame sums; pass partials; frame-sum partials.
 struct glsu_aia {
   int M = 0, Mp = 0, W = 0, H = 0;
   long long N = 0;
@@ -659,16 +684,18 @@ struct glsu_aia {
   void* dmem = nullptr;
   AiaCtl* ctl = nullptr;
   double *delta = nullptr, *Tk = nullptr, *sums_part = nullptr;
-  float *w1 = nullptr, *w2 = nullptr, *dout = nullptr, *part = nullptr;
+  float *w1 = nullptr, *w2 = nullptr, *part = nullptr;
   size_t state_bytes = 0;  // delta + w1 + w2
   void* frames = nullptr;  // host-entry staging (lazy)
   size_t frames_bytes = 0;
   float* phi_dev = nullptr;  // host-entry staging (lazy)
-  // pinned host: the state block's image, the control block, the output shifts
+  // pinned host: the state block's image, the control block, the progress word,
+  // the output shifts
   void* hmem = nullptr;
   double* h_delta = nullptr;
   float *h_w1 = nullptr, *h_w2 = nullptr;
   AiaCtl* h_ctl = nullptr;
+  unsigned long long* h_progress = nullptr;  // done << 32 | completed iterations
   float* h_dout = nullptr;
   hipEvent_t e0 = nullptr, e1 = nullptr;
 };
@@ -710,7 +737,7 @@ extern "C" int glsu_aia_create(glsu_aia** out, int nframes, int width, int heigh
   h->state_bytes = sizeof(double) * M + 2 * sizeof(float) * Mp;
   const size_t bytes = 256 + h->state_bytes + 64 +
                        sizeof(double) * (M + M * h->Gs) +
-                       sizeof(float) * ((5 + 2 * (size_t)KC) * Gtot + M) + 64;
+                       sizeof(float) * (5 + 2 * (size_t)KC) * Gtot + 64;
   auto cleanup = [&](int rc) {
     if (h->dmem) (void)hipFree(h->dmem);
     if (h->hmem) (void)hipHostFree(h->hmem);
@@ -730,11 +757,10 @@ extern "C" int glsu_aia_create(glsu_aia** out, int nframes, int width, int heigh
   p += (h->state_bytes + 63) & ~(size_t)63;
   h->Tk = (double*)p; p += sizeof(double) * M;
   h->sums_part = (double*)p; p += sizeof(double) * M * h->Gs;
-  h->part = (float*)p; p += sizeof(float) * (5 + 2 * (size_t)KC) * Gtot;
-  h->dout = (float*)p;
+  h->part = (float*)p;
   if (hipMemset(h->dmem, 0, bytes) != hipSuccess)
     return cleanup(afail(GLSU_ERR_DEVICE, "hipMemset failed"));
-  const size_t hbytes = ((h->state_bytes + 63) & ~(size_t)63) + 64 + sizeof(float) * M;
+  const size_t hbytes = ((h->state_bytes + 63) & ~(size_t)63) + 128 + sizeof(float) * M;
   if (hipHostMalloc(&h->hmem, hbytes, hipHostMallocDefault) != hipSuccess)
     return cleanup(afail(GLSU_ERR_DEVICE, "hipHostMalloc failed"));
   unsigned char* q = (unsigned char*)h->hmem;
@@ -743,7 +769,8 @@ extern "C" int glsu_aia_create(glsu_aia** out, int nframes, int width, int heigh
   h->h_w2 = h->h_w1 + Mp;
   q += (h->state_bytes + 63) & ~(size_t)63;
   h->h_ctl = (AiaCtl*)q;
-  h->h_dout = (float*)(q + 64);
+  h->h_progress = (unsigned long long*)(q + 64);
+  h->h_dout = (float*)(q + 128);
   for (size_t k = 0; k < Mp; ++k) h->h_w1[k] = h->h_w2[k] = 0.f;
   if (hipEventCreate(&h->e0) != hipSuccess || hipEventCreate(&h->e1) != hipSuccess)
     return cleanup(afail(GLSU_ERR_DEVICE, "hipEventCreate failed"));
@@ -774,7 +801,8 @@ extern "C" int glsu_aia_info(glsu_aia* h, int* blocks, int* chunks, int* frames_
   return GLSU_OK;
 }
 
-// Shifts and first weights to the device (one copy from the pinned image).
+// Shifts and first weights into the pinned image (aia_frame_sums_kernel takes
+// them to the device).
 // Returns the phase-step Cholesky status of the initial shifts.
 static int stage_initial(glsu_aia* h, const double* d0) {
   for (int k = 0; k < h->M; ++k) h->h_delta[k] = d0[k];
@@ -784,7 +812,7 @@ static int stage_initial(glsu_aia* h, const double* d0) {
                  "AIA phase step: the leading minor of order %d is not positive definite; the "
                  "solution could not be computed",
                  info);
-  ATRY(hipMemcpyAsync(h->delta, h->h_delta, h->state_bytes, hipMemcpyHostToDevice, h->s));
+  *h->h_progress = 0;
   return GLSU_OK;
 }
 
@@ -805,7 +833,8 @@ static hipError_t launch_iter(glsu_aia* h, const void* f, int vec, bool first, i
   if (e != hipSuccess) return e;
   hipLaunchKernelGGL((aia_solve_kernel<KC>), dim3(1), dim3(kSolveThreads), solve_smem(h->M), h->s,
                      h->M, h->N, h->G, h->G * nch, h->ctl, h->w1, h->w2, h->delta, h->Tk, h->part,
-                     h->sums_part, first ? h->Gs : 0, max_iter, max_err, err_mode, timing);
+                     h->sums_part, first ? h->Gs : 0, max_iter, max_err, err_mode, timing,
+                     h->h_progress);
   return hipGetLastError();
 }
 
@@ -834,7 +863,9 @@ template <typename T>
 static hipError_t launch_setup(glsu_aia* h, const void* f, int vec, int max_iter, double max_err,
                                int timing) {
   hipLaunchKernelGGL((aia_frame_sums_kernel<T>), dim3(h->Gs, h->M), dim3(kThreads), 0, h->s,
-                     (const T*)f, h->N, vec, h->sums_part, h->ctl, max_iter, max_err, timing);
+                     (const T*)f, h->N, vec, h->sums_part, h->ctl, max_iter, max_err, timing,
+                     (const uint32_t*)h->h_delta, (uint32_t*)h->delta,
+                     (int)(h->state_bytes / sizeof(uint32_t)));
   return hipGetLastError();
 }
 
@@ -845,7 +876,7 @@ static hipError_t launch_final(glsu_aia* h, const void* f, int vec, float* phi) 
   const dim3 g(h->grid_final), b(kThreads);
 #define GLSU_AIA_FINAL(gs)                                                                      \
   hipLaunchKernelGGL((aia_final_kernel<T, gs>), g, b, sm, h->s, (const T*)f, h->M, h->N, vec,  \
-                     h->ctl, h->w1, h->w2, h->delta, phi, h->dout)
+                     h->ctl, h->w1, h->w2, h->delta, phi, h->h_ctl, h->h_dout)
   switch (GS) {
     case 8: GLSU_AIA_FINAL(8); break;
     case 16: GLSU_AIA_FINAL(16); break;
@@ -856,19 +887,38 @@ static hipError_t launch_final(glsu_aia* h, const void* f, int vec, float* phi) 
   return hipGetLastError();
 }
 
+// Waits until `iters` iterations are complete or the loop is over.  The word is
+// read without a call into the runtime; work queued on the stream before this
+// run may take long, so after 2 ms the stream is waited for instead (everything
+// enqueued so far then has reported).
+static hipError_t wait_progress(glsu_aia* h, int iters, bool* over) {
+  const auto t0 = std::chrono::steady_clock::now();
+  for (int spin = 0;; ++spin) {
+    const unsigned long long p = __atomic_load_n(h->h_progress, __ATOMIC_ACQUIRE);
+    *over = (p >> 32) != 0;
+    if (*over || (int)(unsigned)p >= iters) return hipSuccess;
+    if (spin % 64 == 63 && std::chrono::steady_clock::now() - t0 > std::chrono::milliseconds(2)) {
+      const hipError_t e = hipStreamSynchronize(h->s);
+      if (e != hipSuccess) return e;
+      const unsigned long long q = __atomic_load_n(h->h_progress, __ATOMIC_ACQUIRE);
+      *over = (q >> 32) != 0;
+      return *over || (int)(unsigned)q >= iters ? hipSuccess : hipErrorUnknown;
+    }
+  }
+}
+
 template <typename T>
 static hipError_t enqueue_typed(glsu_aia* h, const void* f, int vec, int max_iter, double max_err,
                                 int err_mode, float* phi) {
   hipError_t e = launch_setup<T>(h, f, vec, max_iter, max_err, 0);
   if (e != hipSuccess) return e;
-  for (int it = 0; it < max_iter; ++it) {
-    if (it > 0 && it % kLaunchGroup == 0) {
-      // poll the convergence flag between groups of launches
-      e = hipMemcpyAsync(h->h_ctl, h->ctl, sizeof(AiaCtl), hipMemcpyDeviceToHost, h->s);
-      if (e == hipSuccess) e = hipStreamSynchronize(h->s);
-      if (e != hipSuccess) return e;
-      if (h->h_ctl->done) break;
-    }
+  // the set-up kernel's own test: without it no iteration runs or reports
+  const int n = max_err * 2.0 > max_err ? max_iter : 0;
+  for (int it = 0; it < n; ++it) {
+    bool over = false;
+    e = wait_progress(h, it - kLead + 1, &over);
+    if (e != hipSuccess) return e;
+    if (over) break;
     e = launch_iter_any<T>(h, f, vec, it == 0, max_iter, max_err, err_mode, 0);
     if (e != hipSuccess) return e;
   }
@@ -912,11 +962,12 @@ static int aia_run_dev(glsu_aia* h, const void* d_frames, int dtype, float* delt
     case GLSU_F32: e = enqueue_typed<float>(h, d_frames, vec, max_iter, max_err, err_mode, d_phi); break;
     default: e = enqueue_typed<double>(h, d_frames, vec, max_iter, max_err, err_mode, d_phi); break;
   }
-  if (e != hipSuccess) return afail(GLSU_ERR_DEVICE, "AIA launch failed: %s", hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(h->s);  // nothing may report into the next run
+    return afail(GLSU_ERR_DEVICE, "AIA launch failed: %s", hipGetErrorString(e));
+  }
   ATRY(hipEventRecord(h->e1, h->s));
-  ATRY(hipMemcpyAsync(h->h_ctl, h->ctl, sizeof(AiaCtl), hipMemcpyDeviceToHost, h->s));
-  ATRY(hipMemcpyAsync(h->h_dout, h->dout, sizeof(float) * M, hipMemcpyDeviceToHost, h->s));
-  ATRY(hipStreamSynchronize(h->s));
+  ATRY(hipStreamSynchronize(h->s));  // the final kernel wrote h_ctl and h_dout
   const AiaCtl c = *h->h_ctl;
   if (c.status) {
     const int step = c.status / 10, k = c.status % 10;
@@ -984,12 +1035,18 @@ static int time_iter_typed(glsu_aia* h, const void* f, int vec, int stage, int r
   const int total = stage == 0 ? reps + 1 : 2;  // stage 1: the warm-up leaves done = 0
   hipError_t e = launch_setup<T>(h, f, vec, total, 1.0, 1);
   if (e == hipSuccess) e = launch_iter_any<T>(h, f, vec, true, total, 1.0, 0, 1);  // warm-up
-  if (e != hipSuccess) return afail(GLSU_ERR_DEVICE, "AIA launch failed: %s", hipGetErrorString(e));
+  if (e != hipSuccess) {
+    (void)hipStreamSynchronize(h->s);
+    return afail(GLSU_ERR_DEVICE, "AIA launch failed: %s", hipGetErrorString(e));
+  }
   ATRY(hipEventRecord(h->e0, h->s));
   for (int r = 0; r < reps; ++r) {
     e = stage == 0 ? launch_iter_any<T>(h, f, vec, false, total, 1.0, 0, 1)
                    : launch_pass_any<T>(h, f, vec);
-    if (e != hipSuccess) return afail(GLSU_ERR_DEVICE, "AIA launch failed: %s", hipGetErrorString(e));
+    if (e != hipSuccess) {
+      (void)hipStreamSynchronize(h->s);
+      return afail(GLSU_ERR_DEVICE, "AIA launch failed: %s", hipGetErrorString(e));
+    }
   }
   ATRY(hipEventRecord(h->e1, h->s));
   ATRY(hipMemcpyAsync(h->h_ctl, h->ctl, sizeof(AiaCtl), hipMemcpyDeviceToHost, h->s));
