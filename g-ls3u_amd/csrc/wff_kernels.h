@@ -314,17 +314,24 @@ __device__ __forceinline__ void rows_inv_body(const float2* __restrict__ D,
     float2 nxt[E];
     if (wave < nwx) load_row(nxt, wave);
     for (int k = wave; k < nwx; k += RW) {
+      // this wx's spectrum first: loads return in order, so reading it after
+      // the transform would wait for the next row too (21 planes of 2048 x
+      // 2048: 636 -> 237 us, 3.1 TB/s)
+      float h[E];
+      const float* hx = Hx + (size_t)k * N + lane;
+#pragma unroll
+      for (int j = 0; j < E; ++j) h[j] = hx[j * T];
       float2 v[E];
 #pragma unroll
       for (int j = 0; j < E; ++j) v[j] = nxt[j];
+      __builtin_amdgcn_sched_barrier(0);
       if (k + RW < nwx) load_row(nxt, k + RW);
+      __builtin_amdgcn_sched_barrier(0);
       fft_fwd<P>(v, buf, ctx);
-      const float* hx = Hx + (size_t)k * N + lane;
 #pragma unroll
       for (int j = 0; j < E; ++j) {
-        const float h = hx[j * T];
-        acc[j].x += v[j].x * h;
-        acc[j].y += v[j].y * h;
+        acc[j].x += v[j].x * h[j];
+        acc[j].y += v[j].y * h[j];
       }
     }
   } else {
