@@ -142,21 +142,29 @@ int plan_default(int need, bool t64_only) {
 }
 
 // Column plans of the filter for `items` columns (planes x width): a narrow plan
-// packs several transforms into a wavefront, which pays once the launch has
-// four wavefronts' worth of columns per SIMD; below that it leaves SIMDs empty
-// and every column's chain takes longer on fewer lanes.  Measured, 16 lanes
-// (320 points) against 64 lanes (512 points), 256 rows, 5 planes: 96 columns
-// 28.7 / 16.4 us, 256 29.8 / 19.8, 600 32.4 / 26.9, 900 38.5 / 35.9, 1400 41.5
-// / 46.5; 192 against 256 points, 130 rows: 256 18.8 / 13.7, 900 23.4 / 21.5,
-// 1400 25.7 / 28.6.  The 32-lane plans were slower at every width.
+// packs four transforms into a wavefront, which leaves SIMDs empty and makes
+// every column's chain longer (fewer lanes) until the launch has enough columns.
+// Measured, column kernel, us, 16 lanes / 64 lanes, each with its default
+// workgroups, three filter settings; the lines lie where they cross:
+//   128 / 256 points, 98 rows:  2000 columns 14.1 / 14.0, 2600 14.8 / 16.7, 4090
+//                               15.9 / 19.3, 7000 19.8 / 26.3
+//   192 / 256 points, 130 rows: 2000 18.3 / 13.6, 4090 20.7 / 19.9, 5200 22.3 /
+//                               23.3, 7000 26.3 / 27.4
+//   320 / 512 points, 260 rows: 2000 28.6 / 20.8, 4090 33.5 / 32.1, 4600 35.6 /
+//                               36.5, 7000 40.3 / 45.0
+// Between 4096 and 5200 columns the 192-point plan is within 4 % of the 256-point
+// one on five planes (up to 10 % behind on seven of 132 rows or fewer).  The
+// 32-lane plan of 384 points was slower than 512 points at every width (1280
+// columns 26.7 / 18.4, 12000 92 / 67).
 int plan_default_cols(int need, double items) {
   const int best64 = smallest_plan(need, true);
-  if (best64 >= 0 && items < 4096) return best64;
   int narrow = -1;
   for (const PlanRow& r : kPlanRows)
     if (r.T == 16 && r.N >= need && (narrow < 0 || r.N < plan_row(narrow)->N)) narrow = r.id;
   if (narrow < 0) return best64 >= 0 ? best64 : smallest_plan(need, false);
-  return best64 < 0 || plan_row(narrow)->N < 0.8 * plan_row(best64)->N ? narrow : best64;
+  if (best64 < 0) return narrow;
+  if (plan_row(narrow)->N >= 0.8 * plan_row(best64)->N) return best64;
+  return items < (plan_row(narrow)->N <= 128 ? 2304 : 4096) ? best64 : narrow;
 }
 
 // Window spectra in the order the kernels read them: entry (r, j, lane) holds

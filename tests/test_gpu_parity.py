@@ -169,3 +169,27 @@ def test_default_column_plans_at_their_limits_match_oracle(oracle, W, H, T):
     say(f"   {W}x{H} {w.tuning()} rel={rel:.2e} phase rms={rms:.2e}")
     assert rel < 1e-4
     assert rms < 1e-4
+
+
+@pytest.mark.parametrize("W,H,N", [
+    (460, 98, 256),   # 2300 columns, 128 points needed: still one transform per wavefront
+    (461, 98, 128),   # 2305 columns: four 128-point transforms per wavefront
+    (600, 66, 128),   # 3000 columns, the middle of the range
+    (461, 99, 256),   # 129 points needed: the 192-point plan's line is higher
+])
+def test_default_column_plan_of_short_images_matches_oracle(oracle, W, H, N):
+    """The 128-point narrow plan pays from fewer columns than the longer ones;
+    both sides of its line.  Bars as for the other defaults: FP32 transforms."""
+    rng = np.random.default_rng(W + H)
+    ph = 0.06 * np.arange(W)[None, :] + 0.05 * np.arange(H)[:, None] + rng.normal(0, 0.4, (H, W))
+    f = np.exp(1j * ph).astype(np.complex64)
+    ref = oracle.WFF2(W, H, 10.0, -0.2, 0.2, 0.1)(f.astype(np.complex128))
+    w = glsu.WFT2(W, H, params=glsu.wff_params(10.0, -0.2, 0.2, 0.1))
+    plans = {p["id"]: p for p in glsu.fft_plans()}
+    assert plans[w.tuning()["plany"]]["N"] == N, w.tuning()
+    out = w(torch.from_numpy(f).cuda()).cpu().numpy()
+    rel = np.abs(out - ref).max() / np.abs(ref).max()
+    rms, _ = wrapped_err(np.angle(out), np.angle(ref))
+    say(f"   {W}x{H} {w.tuning()} rel={rel:.2e} phase rms={rms:.2e}")
+    assert rel < 1e-4
+    assert rms < 1e-4
