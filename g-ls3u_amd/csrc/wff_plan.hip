@@ -328,13 +328,28 @@ static hipError_t upload(V*& dptr, const std::vector<V>& h) {
 // waves as long as all of them are resident at once.  Measured, 1 / 2 / 4
 // waves, forward + inverse row kernels of three frames: 256 rows 66 / 58 / 55
 // us, 512 rows 104 / 92 / 89, 768 rows 133 / 120 / 138, 1024 rows 176 / 154 /
-// 194; with 24 points per lane (900 rows) 265 / 330 / 452.
+// 194; of one frame: 450 x 64 22.8 / 19.6 / 18.7, 1200 x 256 47.5 / 39.6 / 37.6,
+// 1200 x 900 59.5 / 52.1 / 65.4.  Longer rows stay whole: one wave per SIMD is
+// resident there, and 900 rows lose by a split (1400 x 900 89 / 108 / 149, 2200
+// x 900 95 / 125); short images of them would gain (1400 x 256 79 / 50 / 49,
+// 2200 x 500 87 / 73) and have no line of their own yet.
 int rows_waves_default(int E, int rows) {
   if (E > 20) return 1;
   int w = 1;
   while (2 * w <= kRowWavesMax && 2 * w * rows <= 2048) w *= 2;
   return w;
 }
+
+// Waves per workgroup of the column kernel.  Workgroups of four waves share one
+// twiddle table best; a launch of few wavefronts (columns / transforms per
+// wavefront) spreads more evenly over the CUs in pairs.  Measured, column
+// kernel, us, 2 / 4 waves a workgroup: 512 points, 1400 wavefronts 19.3 / 20.4,
+// 2150 24.4 / 25.6, 2600 27.5 / 26.8, 3200 30.4 / 31.6, 5200 (1024 x 1024, 1280
+// points) 127 / 121; four 320-point transforms a wavefront, 1300 35.8 / 40.1,
+// 1750 40.3 / 41.2.  Between 2050 and 3072 wavefronts it goes either way by 2 to
+// 5 % with the remainder of the last round; from 1024 points up four waves are
+// ahead there (2050 wavefronts 56.2 / 49.7, 2600 62.8 / 61.7).
+int cols_waves_default(int T, double items) { return items * T < 3072 * 64 ? 2 : 4; }
 
 int wff_plan_geometry(WffPlan& p, int W, int H, double sigx, double wxl, double wxh, double wxi,
                       double sigy, double wyl, double wyh, double wyi, double thr, int planx,
@@ -376,12 +391,9 @@ int wff_plan_geometry(WffPlan& p, int W, int H, double sigx, double wxl, double 
   // rows: one wavefront per transform, up to kRowWavesMax waves per row
   if (rows_waves < 1 || rows_waves > kRowWavesMax) rows_waves = rows_waves_default(px->E, H);
   p.rows_waves = std::min(rows_waves, p.nwx);
-  // columns: workgroups of four waves share one twiddle table best; a launch of
-  // few columns spreads more evenly over the CUs in pairs (256 x 256, 5 planes:
-  // 19.8 / 18.4 us with 4 / 2; 371 x 366, 7 planes 28.2 / 27.1; 1024 x 1024, 5
-  // planes 121 / 127)
-  if (cols_waves == 1 || cols_waves == 2 || cols_waves == 4) p.cols_waves = cols_waves;
-  else if ((double)p.nwx * W * py->T < 3072 * 64) p.cols_waves = 2;
+  if (cols_waves != 1 && cols_waves != 2 && cols_waves != 4)
+    cols_waves = cols_waves_default(py->T, (double)p.nwx * W);
+  p.cols_waves = cols_waves;
   // keep dynamic LDS per workgroup within 64 KiB
   while (p.cols_waves > 1 && plan_smem_bytes(plany, p.cols_waves, true) > 65536) p.cols_waves /= 2;
   while (p.rows_waves > 1 && plan_smem_bytes(planx, p.rows_waves) > 65536) --p.rows_waves;
