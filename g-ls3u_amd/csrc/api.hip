@@ -1103,6 +1103,66 @@ static int batch_alloc_image(BatchImage& im, const WffPlan& cp, const double* ph
   return GLSU_OK;
 }
 
+namespace {
+// One sequence's plans and requested launch shapes.  lx, ly: whether the image
+// fits the live registers of its row / column plan (the kernels compiled for
+// them round slightly differently, and a class shares one choice).
+struct BatchReq {
+  int px, py, cw, rw, lx, ly;
+  bool operator==(const BatchReq& o) const {
+    return px == o.px && py == o.py && cw == o.cw && rw == o.rw && lx == o.lx && ly == o.ly;
+  }
+};
+int live_fit(int plan, int n) {
+  for (const FftPlanInfo& q : fft_plans())
+    if (q.id == plan) return n <= live_regs(q.E) * q.T ? 1 : 0;
+  return 0;
+}
+int plan_lanes(int plan) {
+  for (const FftPlanInfo& q : fft_plans())
+    if (q.id == plan) return q.T;
+  return 0;
+}
+
+// Default column plans of a batch.  One launch carries the columns of every
+// image of a class, so the rule of plan_default_cols takes the columns of them
+// all, not one image's: sixteen images of 256 x 256 (20480 columns) take 154 us
+// a frame with the 16-lane plan, 173 with the 64-lane one, sixty-four 526 and
+// 634.  The images are first grouped by the 64-lane plan; a group whose images
+// all have the same narrow plan takes it by that rule.  Where only some have,
+// they become one more class, three launches a frame more, which pays from
+// 16384 columns: sixteen images of 256 x 256 beside one of 330 rows 184 -> 162
+// us, eight 120 -> 114, but 13160 of the columns of 48 images of 96 to 500 rows
+// 423 -> 444, and all of them in thirty-two images of 96 to 290 rows 193 -> 216.
+void batch_column_plans(std::vector<BatchReq>& req, const glsu_seq_desc* seqs,
+                        const glsu_wff_params* pr, const glsu_tuning* tunings) {
+  const int n = (int)req.size(), sy = (int)std::round(3 * pr->sigma_y);
+  const double nwx = std::floor((pr->wxh - pr->wxl) * (1 / pr->wxi)) + 1;
+  std::vector<BatchReq> wide(req), narrow(req);
+  for (int i = 0; i < n; ++i) {
+    if (tunings && tunings[i].plany >= 0) continue;
+    const int H = seqs[i].height;
+    wide[i].py = plan_default_cols(H + sy, 0);
+    wide[i].ly = live_fit(wide[i].py, H);
+    narrow[i].py = plan_default_cols(H + sy, HUGE_VAL);
+    narrow[i].ly = live_fit(narrow[i].py, H);
+  }
+  for (int i = 0; i < n; ++i) {
+    double items = 0;
+    bool whole = true;
+    for (int k = 0; k < n; ++k)
+      if (wide[k] == wide[i]) {
+        if (narrow[k] == narrow[i]) items += nwx * seqs[k].width;
+        else whole = false;
+      }
+    req[i] = wide[i];
+    if (!(narrow[i] == wide[i]) &&
+        (whole ? plan_default_cols(seqs[i].height + sy, items) == narrow[i].py : items >= 16384))
+      req[i] = narrow[i];
+  }
+}
+}  // namespace
+
 extern "C" int glsu_dpra_batch_create(glsu_dpra_batch** out, const glsu_seq_desc* seqs, int n,
                                       const glsu_wff_params* pr, void* stream,
                                       const glsu_tuning* tunings) {
@@ -1114,15 +1174,7 @@ extern "C" int glsu_dpra_batch_create(glsu_dpra_batch** out, const glsu_seq_desc
     pr = &def;
   }
   // host-side validation of every sequence and its plan choice
-  // lx, ly: whether the image fits the live registers of its row / column
-  // plan (the kernels compiled for them round slightly differently, and a
-  // class shares one choice)
-  struct Req { int px, py, cw, rw, lx, ly; };
-  auto live_fit = [](int plan, int n) {
-    for (const FftPlanInfo& q : fft_plans())
-      if (q.id == plan) return n <= live_regs(q.E) * q.T ? 1 : 0;
-    return 0;
-  };
+  using Req = BatchReq;
   std::vector<Req> req(n);
   for (int i = 0; i < n; ++i) {
     const glsu_seq_desc& d = seqs[i];
@@ -1135,6 +1187,7 @@ extern "C" int glsu_dpra_batch_create(glsu_dpra_batch** out, const glsu_seq_desc
     req[i] = {px, py, t ? t->cols_waves : -1, t ? t->rows_waves : -1, live_fit(px, d.width),
               live_fit(py, d.height)};
   }
+  batch_column_plans(req, seqs, pr, tunings);
   if (int rc = check_device()) return rc;
   auto* h = new glsu_dpra_batch();
   h->n = n;
@@ -1150,9 +1203,7 @@ extern "C" int glsu_dpra_batch_create(glsu_dpra_batch** out, const glsu_seq_desc
   for (int i = 0; i < n; ++i) {
     int c = -1;
     for (size_t k = 0; k < keys.size(); ++k)
-      if (keys[k].px == req[i].px && keys[k].py == req[i].py && keys[k].cw == req[i].cw &&
-          keys[k].rw == req[i].rw && keys[k].lx == req[i].lx && keys[k].ly == req[i].ly)
-        c = (int)k;
+      if (keys[k] == req[i]) c = (int)k;
     if (c < 0) {
       c = (int)keys.size();
       keys.push_back(req[i]);
@@ -1166,14 +1217,19 @@ extern "C" int glsu_dpra_batch_create(glsu_dpra_batch** out, const glsu_seq_desc
     int first = -1;
     for (int i = 0; i < n; ++i)
       if (cls_of[i] == (int)c && first < 0) first = i;
-    if (keys[c].rw < 0) {  // the class's rows share its launches
-      int rows = 0, E = 0;
-      for (int i = 0; i < n; ++i)
-        if (cls_of[i] == (int)c) rows += seqs[i].height;
-      for (const FftPlanInfo& q : fft_plans())
-        if (q.id == keys[c].px) E = q.E;
-      keys[c].rw = rows_waves_default(E, rows);
-    }
+    // the class's rows and columns share its launches
+    int rows = 0, E = 0;
+    double items = 0;
+    for (int i = 0; i < n; ++i)
+      if (cls_of[i] == (int)c) {
+        rows += seqs[i].height;
+        items += seqs[i].width;
+      }
+    items *= std::floor((pr->wxh - pr->wxl) * (1 / pr->wxi)) + 1;
+    for (const FftPlanInfo& q : fft_plans())
+      if (q.id == keys[c].px) E = q.E;
+    if (keys[c].rw < 0) keys[c].rw = rows_waves_default(E, rows);
+    if (keys[c].cw < 0) keys[c].cw = cols_waves_default(plan_lanes(keys[c].py), items);
     std::string err;
     int rc = wff_plan_init(bc.p, seqs[first].width, seqs[first].height, pr->sigma_x, pr->wxl,
                            pr->wxh, pr->wxi, pr->sigma_y, pr->wyl, pr->wyh, pr->wyi, pr->thr,

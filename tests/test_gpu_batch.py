@@ -101,3 +101,31 @@ def test_batch_uneven_workload_shape():
     for i in (0, 5, 11):
         ref = glsu.DPRA(phis[i], 1, tuning=b.tuning(i))(frames[i]).cpu().numpy()
         assert np.array_equal(outs[i].cpu().numpy(), ref)
+
+
+@pytest.mark.parametrize("sizes,expect", [
+    # (lanes per column transform, waves per workgroup) by image
+    ([(256, 256)] * 2, [(64, 2)] * 2),                        # 2560 columns in the launch
+    ([(256, 256)] * 16, [(16, 4)] * 16),                      # 20480 columns
+    ([(96, 98)] * 5, [(16, 2)] * 5),                          # 2400 columns, 128 points
+    ([(300, 400), (470, 400)], [(64, 4)] * 2),                # 1500 + 2350 columns
+    ([(256, 256)] * 12 + [(256, 330)], [(64, 4)] * 13),       # 15360: not worth a class
+    ([(256, 256)] * 13 + [(256, 330)], [(16, 4)] * 13 + [(64, 2)]),  # 16640, 4160 wavefronts
+])
+def test_batch_default_plans_follow_the_columns_of_the_launch(sizes, expect):
+    """The columns of all images of a class run in one launch, so the default
+    column plan and workgroup follow their sum, whatever the order of the
+    list; results as on single handles with those tunings, bit for bit."""
+    plans = {p["id"]: p for p in glsu.fft_plans()}
+    for order in (1, -1):
+        sz, ex = sizes[::order], expect[::order]
+        frames, phis = _inputs(sz, 2, seed0=900)
+        b = glsu.DPRABatch(phis, 1)
+        got = [(plans[b.tuning(i)["plany"]]["T"], b.tuning(i)["cols_waves"])
+               for i in range(len(sz))]
+        say(f"[batch plans] {len(sz)} sequences {got} classes={b.info()['classes']}")
+        assert got == ex
+        outs = b(frames)
+        for i in (0, len(sz) - 1):
+            ref = glsu.DPRA(phis[i], 1, tuning=b.tuning(i))(frames[i])
+            assert torch.equal(outs[i], ref)
