@@ -5,7 +5,9 @@ Each sequence behaves as its own DPRA_CPU / DPRA_CUDAF object
 and rr, then driven by operator()(frames, dPhi_Sum, time).  The batch runs all
 of them together on the device (one least-squares launch over all images and
 one launch per WFF2 stage per FFT-plan group, per frame) and matches
-glsu.DPRA on each sequence bit for bit when both use the same tuning.
+glsu.DPRA on each sequence bit for bit when both use the same tuning.  Default
+tunings follow the rows and columns of all sequences that share a launch: give
+full tunings where a sequence's rounding must not change with its company.
 """
 import ctypes
 

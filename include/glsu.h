@@ -248,7 +248,12 @@ typedef struct glsu_seq_desc {
   const double *phi0;      /* host, height*width initial phase */
 } glsu_seq_desc;
 typedef struct glsu_dpra_batch glsu_dpra_batch;
-/* tunings: n entries (one per sequence) or NULL for the defaults. */
+/* tunings: n entries (one per sequence) or NULL for the defaults.  Defaults
+ * (also of single fields left at -1) follow the rows and columns of all
+ * sequences that share a launch, so a sequence's default plans, and with them
+ * its rounding, can differ from those of a handle of its own and change with
+ * the other sequences of the batch; glsu_dpra_batch_get_tuning tells them, and
+ * a tuning given in full does not depend on the others. */
 int glsu_dpra_batch_create(glsu_dpra_batch **out, const glsu_seq_desc *seqs, int n,
                            const glsu_wff_params *p, void *hip_stream,
                            const glsu_tuning *tunings);

@@ -129,3 +129,21 @@ def test_batch_default_plans_follow_the_columns_of_the_launch(sizes, expect):
         for i in (0, len(sz) - 1):
             ref = glsu.DPRA(phis[i], 1, tuning=b.tuning(i))(frames[i])
             assert torch.equal(outs[i], ref)
+
+
+def test_full_tunings_make_a_sequence_independent_of_the_others():
+    """A sequence with the tuning of a handle of its own size gives that
+    handle's results bit for bit, alone or beside any others."""
+    sizes = [(256, 256)] * 16 + [(300, 211)]
+    frames, phis = _inputs(sizes, 3, seed0=1100)
+    own = []
+    for i in (0, 16):
+        d = glsu.DPRA(phis[i], 1)
+        own.append((d.tuning(), d(frames[i])))
+    tunings = [own[0][0]] * 16 + [own[1][0]]
+    assert glsu.DPRABatch(phis, 1).tuning(0)["plany"] != own[0][0]["plany"]
+    full = glsu.DPRABatch(phis, 1, tunings=tunings)(frames)
+    pair = glsu.DPRABatch([phis[0], phis[16]], 1,
+                          tunings=[own[0][0], own[1][0]])([frames[0], frames[16]])
+    for k, i in enumerate((0, 16)):
+        assert torch.equal(full[i], own[k][1]) and torch.equal(pair[k], own[k][1])
