@@ -1033,7 +1033,6 @@ struct glsu_dpra_batch {
   int* h_frame = nullptr;       // pinned
   int ntiles = 0, grid_ls = 0;
   std::map<int, std::pair<hipGraph_t, hipGraphExec_t>> graphs;  // by frame dtype
-  std::map<int, bool> seen;  // frame dtypes of earlier calls
   hipEvent_t e0 = nullptr, e1 = nullptr;
   // Side streams: the classes' WFF2 chains are independent between the
   // threshold and the frame's end.  Where no class gives the column kernel more
@@ -1373,12 +1372,6 @@ extern "C" int glsu_dpra_batch_run(glsu_dpra_batch* h, const void* const* frames
                          hipMemcpyHostToDevice, h->s));
   HIP_TRY(hipMemcpyAsync(h->d_frame, h->h_frame, sizeof(int), hipMemcpyHostToDevice, h->s));
   if (ms) HIP_TRY(hipEventRecord(h->e0, h->s));
-  // the first call of a few frames launches them directly: capturing and
-  // instantiating the graph (about 0.3 ms) costs more than replaying it saves
-  // there (13 us a frame)
-  bool& seen = h->seen[dtype];
-  if (use_graph && !seen && nframes < 16) use_graph = 0;
-  seen = true;
   if (use_graph) {
     auto it = h->graphs.find(dtype);
     if (it == h->graphs.end()) {
