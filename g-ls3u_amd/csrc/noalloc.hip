@@ -66,8 +66,9 @@ int fail_noalloc(int code, const char* msg) {
 }  // namespace
 
 // One WFF-mode WFT2 (init + compute) of a height x width complex64 field, with
-// the plans and launch shapes glsu_wft2_create picks by default; no handle,
-// no allocation.  See include/glsu.h.
+// the plans and launch shapes glsu_wft2_create picks by default (the shortest
+// column plan where the spectra of that one do not fit); no handle, no
+// allocation.  See include/glsu.h.
 extern "C" int glsu_wft2_compute_noalloc(int width, int height, const glsu_wff_params* pr,
                                          const void* d_f, void* d_filtered, void* hip_stream) {
   if (!pr || !d_f || !d_filtered) return fail_noalloc(GLSU_ERR_ARG, "null argument");
@@ -81,36 +82,43 @@ extern "C" int glsu_wft2_compute_noalloc(int width, int height, const glsu_wff_p
   if (W + 2 * sx > 4096 || H + 2 * sy > 4096)
     return fail_noalloc(GLSU_ERR_PADDING, "FFT padding is out of range [4096]");
   const double nwx = std::floor((pr->wxh - pr->wxl) * (1 / pr->wxi)) + 1;
-  const int planx = plan_default(W + sx, true), plany = plan_default_cols(H + sy, nwx * W);
+  const int planx = plan_default(W + sx, true), shortest = plan_default(H + sy, false);
+  int plany = plan_default_cols(H + sy, nwx * W);
   if (planx < 0 || plany < 0)
     return fail_noalloc(GLSU_ERR_PADDING, "no compiled FFT length covers the size + half window");
   WffPlan p;
-  const char* err = nullptr;
-  if (wff_plan_geometry(p, W, H, pr->sigma_x, pr->wxl, pr->wxh, pr->wxi, pr->sigma_y, pr->wyl,
-                        pr->wyh, pr->wyi, pr->thr, planx, plany, -1, -1, &err))
-    return fail_noalloc(GLSU_ERR_ARG, err ? err : "invalid plan");
-  // carve the scratch array: windows, spectra, twiddles, threshold, partial
-  // sums, then the two plane sets
-  size_t off = 0;
-  auto take = [&](size_t bytes) {
-    const size_t o = off;
-    off = align256(off + bytes);
-    return o;
-  };
-  const size_t o_gx = take(sizeof(double) * (2 * p.sx + 1));
-  const size_t o_gy = take(sizeof(double) * (2 * p.sy + 1));
-  const size_t o_hx = take(sizeof(float) * (size_t)p.nwx * p.Nx);
-  const size_t o_hy = take(sizeof(float) * (size_t)p.nwy * p.Ny);
-  const size_t o_tx = take(sizeof(float2) * (size_t)p.Nx);
-  const size_t o_ty = take(sizeof(float2) * (size_t)p.Ny);
-  const size_t o_thr = take(sizeof(float));
-  const size_t o_red = take(sizeof(float) * 256);
-  const size_t o_a = take(sizeof(float2) * p.plane_elems * p.nwx);
-  const size_t o_d = take(sizeof(float2) * p.plane_elems * p.nwx);
-  if (off > kScratchBytes)
-    return fail_noalloc(GLSU_ERR_UNSUPPORTED,
-                        "field too large for the no-allocation scratch (96 MiB: e.g. 1024x1024 "
-                        "with up to 5 wx values)");
+  size_t o_gx, o_gy, o_hx, o_hy, o_tx, o_ty, o_thr, o_red, o_a, o_d, off;
+  for (;;) {
+    const char* err = nullptr;
+    if (wff_plan_geometry(p, W, H, pr->sigma_x, pr->wxl, pr->wxh, pr->wxi, pr->sigma_y, pr->wyl,
+                          pr->wyh, pr->wyi, pr->thr, planx, plany, -1, -1, &err))
+      return fail_noalloc(GLSU_ERR_ARG, err ? err : "invalid plan");
+    // carve the scratch array: windows, spectra, twiddles, threshold, partial
+    // sums, then the two plane sets
+    off = 0;
+    auto take = [&](size_t bytes) {
+      const size_t o = off;
+      off = align256(off + bytes);
+      return o;
+    };
+    o_gx = take(sizeof(double) * (2 * p.sx + 1));
+    o_gy = take(sizeof(double) * (2 * p.sy + 1));
+    o_hx = take(sizeof(float) * (size_t)p.nwx * p.Nx);
+    o_hy = take(sizeof(float) * (size_t)p.nwy * p.Ny);
+    o_tx = take(sizeof(float2) * (size_t)p.Nx);
+    o_ty = take(sizeof(float2) * (size_t)p.Ny);
+    o_thr = take(sizeof(float));
+    o_red = take(sizeof(float) * 256);
+    o_a = take(sizeof(float2) * p.plane_elems * p.nwx);
+    o_d = take(sizeof(float2) * p.plane_elems * p.nwx);
+    if (off <= kScratchBytes) break;
+    // a very fine wy grid: the spectra of the shortest column plan may still fit
+    if (plany == shortest)
+      return fail_noalloc(GLSU_ERR_UNSUPPORTED,
+                          "field too large for the no-allocation scratch (96 MiB: e.g. 1024x1024 "
+                          "with up to 5 wx values)");
+    plany = shortest;
+  }
   unsigned char* base = nullptr;
   if (int rc = scratch_ptr(&base)) return rc;
   p.d_Hx = (float*)(base + o_hx);

@@ -76,3 +76,23 @@ def test_noalloc_rejects_fields_beyond_the_scratch():
                                               ctypes.c_void_p(f.data_ptr()),
                                               ctypes.c_void_p(f.data_ptr()), None)
     assert rc == glsu._lib.ERR_PADDING
+
+
+def test_noalloc_takes_the_shortest_plan_where_the_default_does_not_fit():
+    """49999 wy values at 271 padded rows: the 512-point spectra that the
+    default plan of four columns would need take 98 MiB, the 320-point ones 61.
+    Against a handle with that plan, bar as above."""
+    W, H, nwy = 4, 270, 50000
+    step = 2.0 / nwy
+    params = glsu.wff_params(0.4, -1.0, -1.0 + (nwy - 1.5) * step, step, thr=0.0)
+    params.wxl, params.wxh, params.wxi = 0.0, 0.1, 0.2  # one wx
+    f = _field(W, H, 3)
+    out = torch.full_like(f, complex(float("nan"), float("nan")))
+    say(f"[noalloc] {W}x{H}, {nwy} wy values")
+    assert _noalloc(f, params, out) == glsu._lib.OK, glsu.lib().glsu_last_error()
+    plan = min((p["N"], p["id"]) for p in glsu.fft_plans() if p["N"] >= H + 1)[1]
+    ref = glsu.WFT2(W, H, params=params, plany=plan)(f)
+    a, b = out.cpu().numpy(), ref.cpu().numpy()
+    rel = float(np.abs(a - b).max() / np.abs(b).max())
+    say(f"   rel {rel:.2e}")
+    assert np.abs(b).max() > 0 and rel <= 1e-6
