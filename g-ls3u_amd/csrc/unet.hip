@@ -41,6 +41,7 @@ struct Acts {  // activations and gradients for one (n, H, W)
   float2* out = nullptr;
   float* loss = nullptr;
   float* ws = nullptr;  // partial sums of one layer's weight gradient (backward only)
+  int cus = 0;          // CU count that ws is sized for
 };
 }  // namespace
 
@@ -174,28 +175,31 @@ static int forward(glsu_unet* h, const float2* x, float2* out, int n, int H, int
 static int grads_alloc(glsu_unet* h, int n, int H, int W) {
   Acts& a = h->a;
   if (a.ws) return GLSU_OK;
+  const int cus = unet_device_cus();
+  if (cus < 1) return ufail(GLSU_ERR_DEVICE, "device query failed");
   std::vector<std::pair<void**, size_t>> want;
   const size_t P = (size_t)n * H * W;
-  size_t m = std::max(unet_conv3_in_dw_floats(n, H, h->C(0)),
-                      unet_conv1_out_bwd_floats((long)P, h->C(0)));
+  size_t m = std::max(unet_conv3_in_dw_floats(n, H, h->C(0), cus),
+                      unet_conv1_out_bwd_floats((long)P, h->C(0), cus));
   for (int l = 0; l < h->levels; ++l) {
     const int Hl = H >> l, Wl = W >> l, C = h->C(l);
     const size_t px = (size_t)n * Hl * Wl, b = px * C * sizeof(__bf16);
     want.push_back({(void**)&a.ge[l], b});
     want.push_back({(void**)&a.gea[l], b});
-    m = std::max(m, unet_conv3_dw_floats(C, C, 0, n, Hl, Wl));
-    if (l > 0) m = std::max(m, unet_conv3_dw_floats(C, h->C(l - 1), 0, n, Hl, Wl));
+    m = std::max(m, unet_conv3_dw_floats(C, C, 0, n, Hl, Wl, cus));
+    if (l > 0) m = std::max(m, unet_conv3_dw_floats(C, h->C(l - 1), 0, n, Hl, Wl, cus));
     if (l < h->levels - 1) {
       want.push_back({(void**)&a.gp[l], b / 4});
       want.push_back({(void**)&a.gd[l], b});
       want.push_back({(void**)&a.gda[l], b});
       want.push_back({(void**)&a.gcat[l], px * (C + h->C(l + 1)) * sizeof(__bf16)});
-      m = std::max(m, unet_conv3_dw_floats(C, C, h->C(l + 1), n, Hl, Wl));
+      m = std::max(m, unet_conv3_dw_floats(C, C, h->C(l + 1), n, Hl, Wl, cus));
     }
   }
   want.push_back({(void**)&a.out, P * sizeof(float2)});
   want.push_back({(void**)&a.loss, sizeof(float)});
   want.push_back({(void**)&a.ws, m * sizeof(float)});
+  a.cus = cus;
   return arena_alloc(a, want);
 }
 
@@ -207,7 +211,7 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
   const long P = (long)n * H * W;
   Layer& o = h->out();
   UTRY(unet_conv1_out_bwd(a.d[0], a.out, u, o.w, a.gd[0], o.gw, o.gb, a.loss, a.ws, P,
-                          h->C(0), s));
+                          h->C(0), a.cus, s));
   // decoder, top level first; gd[l]: gradient at the pre-activation of d_l
   __bf16* ge_top = nullptr;
   for (int l = 0; l <= Lv - 2; ++l) {
@@ -216,10 +220,11 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
     Layer& la = h->dec(l, 0);
     Layer& lb = h->dec(l, 1);
     const __bf16* low = (l + 1 <= Lv - 2) ? a.d[l + 1] : a.e[Lv - 1];
-    UTRY(unet_conv3_dw(a.gd[l], Cl, a.da[l], Cl, nullptr, 0, lb.gw, lb.gb, a.ws, n, Hl, Wl, s));
+    UTRY(unet_conv3_dw(a.gd[l], Cl, a.da[l], Cl, nullptr, 0, lb.gw, lb.gb,
+                       a.ws, n, Hl, Wl, a.cus, s));
     UTRY(unet_conv3(a.gd[l], Cl, nullptr, 0, lb.wt, nullptr, a.da[l], a.gda[l], n, Hl, Wl, Cl, 1,
                     s));
-    UTRY(unet_conv3_dw(a.gda[l], Cl, a.e[l], Cl, low, Cn, la.gw, la.gb, a.ws, n, Hl, Wl, s));
+    UTRY(unet_conv3_dw(a.gda[l], Cl, a.e[l], Cl, low, Cn, la.gw, la.gb, a.ws, n, Hl, Wl, a.cus, s));
     UTRY(unet_conv3(a.gda[l], Cl, nullptr, 0, la.wt, nullptr, nullptr, a.gcat[l], n, Hl, Wl,
                     Cl + Cn, 1, s));
     __bf16* gl = (l + 1 <= Lv - 2) ? a.gd[l + 1] : a.ge[Lv - 1];
@@ -233,15 +238,17 @@ static int backward(glsu_unet* h, const float2* x, const float2* u, int n, int H
     const int Cl = h->C(l);
     Layer& la = h->enc(l, 0);
     Layer& lb = h->enc(l, 1);
-    UTRY(unet_conv3_dw(a.ge[l], Cl, a.ea[l], Cl, nullptr, 0, lb.gw, lb.gb, a.ws, n, Hl, Wl, s));
+    UTRY(unet_conv3_dw(a.ge[l], Cl, a.ea[l], Cl, nullptr, 0, lb.gw, lb.gb,
+                       a.ws, n, Hl, Wl, a.cus, s));
     UTRY(unet_conv3(a.ge[l], Cl, nullptr, 0, lb.wt, nullptr, a.ea[l], a.gea[l], n, Hl, Wl, Cl, 1,
                     s));
     if (l == 0) {
-      UTRY(unet_conv3_in_dw(x, a.gea[0], la.gw, la.gb, a.ws, n, H, W, Cl, s));
+      UTRY(unet_conv3_in_dw(x, a.gea[0], la.gw, la.gb, a.ws, n, H, W, Cl, a.cus, s));
       break;
     }
     const int Cp = h->C(l - 1);
-    UTRY(unet_conv3_dw(a.gea[l], Cl, a.p[l - 1], Cp, nullptr, 0, la.gw, la.gb, a.ws, n, Hl, Wl, s));
+    UTRY(unet_conv3_dw(a.gea[l], Cl, a.p[l - 1], Cp, nullptr, 0, la.gw, la.gb,
+                       a.ws, n, Hl, Wl, a.cus, s));
     UTRY(unet_conv3(a.gea[l], Cl, nullptr, 0, la.wt, nullptr, nullptr, a.gp[l - 1], n, Hl, Wl, Cp,
                     1, s));
     UTRY(unet_pool_bwd(a.e[l - 1], a.gp[l - 1], a.gcat[l - 1], Cp + Cl, a.ge[l - 1], n, H >> (l - 1),

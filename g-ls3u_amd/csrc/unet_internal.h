@@ -13,24 +13,27 @@ namespace glsu {
 hipError_t unet_conv3(const __bf16* X1, int C1, const __bf16* X2, int C2, const __bf16* Wt,
                       const float* bias, const __bf16* mask, __bf16* Y, int n, int H, int W,
                       int Cout, int mode, hipStream_t s, __bf16* pool = nullptr);
+// CUs of the current device, 0 on error.  The gradient launchers and the sizes of
+// their scratch take the number from the caller, who keeps one for both.
+int unet_device_cus();
 // dW [Cout][9][Cin] = weight gradient, db [Cout] = bias gradient (FP32, summed
 // in a fixed order); ws: unet_conv3_dw_floats() floats of scratch
-size_t unet_conv3_dw_floats(int Cout, int C1, int C2, int n, int H, int W);
+size_t unet_conv3_dw_floats(int Cout, int C1, int C2, int n, int H, int W, int cus);
 hipError_t unet_conv3_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
-                         int C2, float* dW, float* db, float* ws, int n, int H, int W,
+                         int C2, float* dW, float* db, float* ws, int n, int H, int W, int cus,
                          hipStream_t s);
 hipError_t unet_conv3_in(const float2* x, const float* w, const float* b, __bf16* Y, int n,
                          int H, int W, int C0, hipStream_t s);
 // input and output layer gradients, written whole; ws: *_floats() of scratch
-size_t unet_conv3_in_dw_floats(int n, int H, int C0);
+size_t unet_conv3_in_dw_floats(int n, int H, int C0, int cus);
 hipError_t unet_conv3_in_dw(const float2* x, const __bf16* dY, float* dW, float* db, float* ws,
-                            int n, int H, int W, int C0, hipStream_t s);
+                            int n, int H, int W, int C0, int cus, hipStream_t s);
 hipError_t unet_conv1_out(const __bf16* d, const float2* x, const float* w, const float* b,
                           float2* out, long P, int C0, hipStream_t s);
 hipError_t unet_conv1_out_bwd(const __bf16* d, const float2* out, const float2* u,
                               const float* w, __bf16* dd, float* dW, float* db, float* loss,
-                              float* ws, long P, int C0, hipStream_t s);
-size_t unet_conv1_out_bwd_floats(long P, int C0);
+                              float* ws, long P, int C0, int cus, hipStream_t s);
+size_t unet_conv1_out_bwd_floats(long P, int C0, int cus);
 hipError_t unet_maxpool2(const __bf16* x, __bf16* y, int n, int H, int W, int C, hipStream_t s);
 hipError_t unet_pool_bwd(const __bf16* e, const __bf16* gp, const __bf16* gskip, int Cs,
                          __bf16* ge, int n, int H, int W, int C, hipStream_t s);

@@ -13,6 +13,7 @@
 #include "unet_internal.h"
 
 #include <algorithm>
+#include <atomic>
 
 namespace glsu {
 
@@ -1457,6 +1458,21 @@ __global__ __launch_bounds__(256) void weights_to_bf16_kernel(const float* __res
 // ======================================================== host launchers
 static unsigned blocks(long work, int per = 256) { return (unsigned)((work + per - 1) / per); }
 
+// CUs of the current device (0 on error); callable from several threads.
+int unet_device_cus() {
+  constexpr int kDevices = 64;
+  static std::atomic<int> cus[kDevices] = {};
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kDevices) return 0;
+  int v = cus[dev].load(std::memory_order_relaxed);
+  if (v == 0) {
+    if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
+      return 0;
+    cus[dev].store(v, std::memory_order_relaxed);
+  }
+  return v;
+}
+
 hipError_t unet_conv3(const __bf16* X1, int C1, const __bf16* X2, int C2, const __bf16* Wt,
                       const float* bias, const __bf16* mask, __bf16* Y, int n, int H, int W,
                       int Cout, int mode, hipStream_t s, __bf16* pool) {
@@ -1467,13 +1483,8 @@ hipError_t unet_conv3(const __bf16* X1, int C1, const __bf16* X2, int C2, const 
   const int cob = (Cout + nco - 1) / nco;
   if (nco == 32 && H % kRTileH == 0) {
     // persistent 8-row kernel: two workgroups per CU (64 KB LDS, <= 256 registers)
-    static int cus = 0;
-    if (cus == 0) {
-      int dev = 0;
-      if (hipGetDevice(&dev) != hipSuccess ||
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return hipErrorInvalidValue;
-    }
+    const int cus = unet_device_cus();
+    if (cus < 1) return hipErrorInvalidValue;
     const int rtiles = n * (H / kRTileH) * ((W + RowsConv<32>::TW - 1) / RowsConv<32>::TW);
     dim3 grid(std::min(rtiles, std::max(1, 2 * cus / cob)), cob);
     if (mode == 0)
@@ -1488,13 +1499,8 @@ hipError_t unet_conv3(const __bf16* X1, int C1, const __bf16* X2, int C2, const 
     // one 8-wave workgroup per CU: weights resident up to 64 input channels;
     // above that, for the forward pass, streamed per chunk where the tiles fill
     // every CU
-    static int cus = 0;
-    if (cus == 0) {
-      int dev = 0;
-      if (hipGetDevice(&dev) != hipSuccess ||
-          hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return hipErrorInvalidValue;
-    }
+    const int cus = unet_device_cus();
+    if (cus < 1) return hipErrorInvalidValue;
     const int xt = n * (H / kXTileH) * ((W + kXTileW - 1) / kXTileW);
     const bool resident = C1 + C2 <= kXMaxCin;
     if (resident || (mode == 0 && xt * cob >= cus)) {
@@ -1574,18 +1580,6 @@ static hipError_t launch_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1
   return hipGetLastError();
 }
 
-static int device_cus() {
-  static int cus = 0;
-  if (cus == 0) {
-    int dev = 0, v = 0;
-    if (hipGetDevice(&dev) != hipSuccess ||
-        hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-      return 0;
-    cus = v;
-  }
-  return cus;
-}
-
 // The widest channel tile that divides the layer: 64 x 64 reads each operand
 // for two blocks; narrower layers share the workgroup's waves over strips.
 static int dw_tile(int Cout, int C1, int C2) {
@@ -1593,8 +1587,8 @@ static int dw_tile(int Cout, int C1, int C2) {
   return C1 % 64 || C2 % 64 ? 1 : 2;
 }
 
-size_t unet_conv3_dw_floats(int Cout, int C1, int C2, int n, int H, int W) {
-  const int cus = std::max(1, device_cus()), Cin = C1 + C2;
+size_t unet_conv3_dw_floats(int Cout, int C1, int C2, int n, int H, int W, int cus) {
+  const int Cin = C1 + C2;
   DwSplit d;
   switch (dw_tile(Cout, C1, C2)) {
     case 2: d = dw_split<2, 2, 2, 2>(Cout, Cin, n, H, W, cus); break;
@@ -1605,11 +1599,10 @@ size_t unet_conv3_dw_floats(int Cout, int C1, int C2, int n, int H, int W) {
 }
 
 hipError_t unet_conv3_dw(const __bf16* dY, int Cout, const __bf16* X1, int C1, const __bf16* X2,
-                         int C2, float* dW, float* db, float* ws, int n, int H, int W,
+                         int C2, float* dW, float* db, float* ws, int n, int H, int W, int cus,
                          hipStream_t s) {
-  if ((C1 % 32) || (C2 % 32) || (Cout % 32) || (C2 && ((H | W) & 1))) return hipErrorInvalidValue;
-  const int cus = device_cus();
-  if (cus < 1) return hipErrorInvalidValue;
+  if ((C1 % 32) || (C2 % 32) || (Cout % 32) || (C2 && ((H | W) & 1)) || cus < 1)
+    return hipErrorInvalidValue;
   switch (dw_tile(Cout, C1, C2)) {
     case 2:
       return launch_dw<2, 2, 2, 2>(dY, Cout, X1, C1, X2, C2, dW, db, ws, n, H, W, cus, s);
@@ -1629,16 +1622,16 @@ hipError_t unet_conv3_in(const float2* x, const float* w, const float* b, __bf16
 }
 
 // workgroups of conv3_in_dw_kernel (two per CU, rows dealt round robin)
-static int in_dw_wgs(long rows, int C0) {
-  return (int)std::max(1L, std::min<long>(rows, 2L * device_cus() / (C0 / 32)));
+static int in_dw_wgs(long rows, int C0, int cus) {
+  return (int)std::max(1L, std::min<long>(rows, 2L * cus / (C0 / 32)));
 }
-size_t unet_conv3_in_dw_floats(int n, int H, int C0) {
-  return (size_t)in_dw_wgs((long)n * H, C0) * C0 * 19;
+size_t unet_conv3_in_dw_floats(int n, int H, int C0, int cus) {
+  return (size_t)in_dw_wgs((long)n * H, C0, cus) * C0 * 19;
 }
 hipError_t unet_conv3_in_dw(const float2* x, const __bf16* dY, float* dW, float* db, float* ws,
-                            int n, int H, int W, int C0, hipStream_t s) {
-  if (C0 % 32) return hipErrorInvalidValue;
-  const int wgs = in_dw_wgs((long)n * H, C0);
+                            int n, int H, int W, int C0, int cus, hipStream_t s) {
+  if (C0 % 32 || cus < 1) return hipErrorInvalidValue;
+  const int wgs = in_dw_wgs((long)n * H, C0, cus);
   hipLaunchKernelGGL(conv3_in_dw_kernel, dim3(wgs, C0 / 32), dim3(512), 0, s, x, dY, ws, n, H, W,
                      C0);
   const hipError_t e = hipGetLastError();
@@ -1655,17 +1648,17 @@ hipError_t unet_conv1_out(const __bf16* d, const float2* x, const float* w, cons
 }
 
 // workgroups of conv1_out_bwd_kernel (eight per CU walk the pixels)
-static int out_bwd_wgs(long P, int C0) {
-  return (int)std::max(1L, std::min<long>((P + 63) / 64, 8L * device_cus() / (C0 / 32)));
+static int out_bwd_wgs(long P, int C0, int cus) {
+  return (int)std::max(1L, std::min<long>((P + 63) / 64, 8L * cus / (C0 / 32)));
 }
-size_t unet_conv1_out_bwd_floats(long P, int C0) {
-  return (size_t)out_bwd_wgs(P, C0) * (2 * C0 + 3);
+size_t unet_conv1_out_bwd_floats(long P, int C0, int cus) {
+  return (size_t)out_bwd_wgs(P, C0, cus) * (2 * C0 + 3);
 }
 hipError_t unet_conv1_out_bwd(const __bf16* d, const float2* out, const float2* u,
                               const float* w, __bf16* dd, float* dW, float* db, float* loss,
-                              float* ws, long P, int C0, hipStream_t s) {
-  if (C0 % 32) return hipErrorInvalidValue;
-  const int wgs = out_bwd_wgs(P, C0);
+                              float* ws, long P, int C0, int cus, hipStream_t s) {
+  if (C0 % 32 || cus < 1) return hipErrorInvalidValue;
+  const int wgs = out_bwd_wgs(P, C0, cus);
   hipLaunchKernelGGL(conv1_out_bwd_kernel, dim3(wgs, C0 / 32), dim3(256), 0, s, d, out, u, w, dd,
                      ws, P, C0);
   const hipError_t e = hipGetLastError();
