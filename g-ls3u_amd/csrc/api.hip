@@ -1498,8 +1498,9 @@ extern "C" int glsu_dpra_frame_learned(glsu_dpra* h, glsu_unet* net, const void*
   if (it == h->wins.end()) {
     WffPlan wp;
     std::string err;
-    // same plan rule as the public constructors (row plans use 64 lanes)
-    const int px = default_plan(Ww + p.sx, true), py = default_plan(Hw + p.sy, false);
+    // the same default plans as a WFT2 handle of the window's size
+    const int px = default_plan(Ww + p.sx, true);
+    const int py = plan_default_cols(Hw + p.sy, (double)p.nwx * Ww);
     if (px < 0 || py < 0) return fail(GLSU_ERR_ARG, "no FFT plan for the spot-check window");
     int rc = wff_plan_init(wp, Ww, Hw, p.sigx, p.wxl, p.wxh, p.wxi, p.sigy, p.wyl, p.wyh, p.wyi,
                            -1.0, px, py, -1, -1, err);
