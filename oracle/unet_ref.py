@@ -70,7 +70,7 @@ def conv3_bwd(x, w, g):
     gw = np.zeros_like(w)
     for dy in range(3):
         for dx in range(3):
-            gw[:, dy, dx, :] = np.einsum("nhwo,nhwi->oi", g, xp[:, dy:dy + H, dx:dx + W])
+            gw[:, dy, dx, :] = np.tensordot(g, xp[:, dy:dy + H, dx:dx + W], axes=([0, 1, 2],) * 2)
             gx[:, dy:dy + H, dx:dx + W] += g @ w[:, dy, dx, :]
     return gx[:, 1:-1, 1:-1], gw, g.sum(axis=(0, 1, 2))
 

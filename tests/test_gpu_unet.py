@@ -11,6 +11,8 @@ gradient is a sum over pixels of random-phase inputs that cancels to ~1/10 of
 its terms, which amplifies the BF16 error it inherits from the whole backward
 pass; it is held to direction (cosine > 0.98) and a 0.2 relative norm, which
 a wrong tap, channel or sign would fail by far."""
+import math
+
 import numpy as np
 import pytest
 
@@ -261,3 +263,123 @@ def test_gradients_at_strip_and_chunk_edges(levels, base, n, H, W):
             assert rel < 0.2 and cos > 0.98, k
         else:
             assert rel < 6e-2, k
+
+
+@pytest.mark.parametrize("levels,base,H,W", [
+    (2, 32, 16, 130),   # 130 = 128 + 2 pixels of a strip group, 2 * 64 + 2 of the input layer's lanes
+    (2, 32, 16, 260),   # the half-resolution layers have the 2-pixel remainder too
+    (2, 64, 16, 66),    # 64-channel tiles: strips of 64 pixels
+    (2, 96, 16, 130),   # channel counts that only 32 divides
+])
+def test_gradients_of_a_signal_in_the_last_columns(levels, base, H, W):
+    """The target differs from the output in the last two columns only, so
+    every layer's gradient comes from the part strips there.  Bar: a lost
+    remainder changes the layer it belongs to by at least 0.48 in norm (the
+    FP64 reference with those columns of the layer's gradient left out); BF16
+    rounding of activations and gradients, emulated in the reference, by at
+    most 0.16 over four seeds (few pixels: ReLU and pooling decisions weigh
+    more than in the tests above)."""
+    net, ref = _net_and_ref(seed=31, levels=levels, base=base)
+    x, _ = _inputs(1, H, W, seed=32)
+    rng = np.random.default_rng(33)
+    delta = np.zeros((1, H, W), np.complex64)
+    delta[:, :, -2:] = rng.normal(0, 0.5, (1, H, 2)) + 1j * rng.normal(0, 0.5, (1, H, 2))
+    xg = torch.from_numpy(x).cuda()
+    net.loss_grad(xg, net.forward(xg) + torch.from_numpy(delta).cuda())
+    g = net.grads()
+    _, gr = U.loss_and_grads(ref, _c2(x), U.forward(ref, _c2(x), levels) + _c2(delta), levels)
+    for k in gr:
+        a, b = g[k].astype(np.float64).ravel(), gr[k].ravel()
+        rel = np.linalg.norm(a - b) / np.linalg.norm(b)
+        say(f"   {k:8s} rel err {rel:.2e}")
+        assert rel < 0.3, k
+
+
+def test_gradients_with_several_strips_per_workgroup():
+    """288 and 576 channels on 8 x 832 pixels: more strips than workgroups a
+    channel tile, so each workgroup walks several, for all three tile shapes
+    (32 x 32: 288 -> 288 and 864 -> 288, 64 x 32: 288 -> 576, 64 x 64: 576 ->
+    576).  Bars as above."""
+    levels, base, H, W = 2, 288, 8, 832
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    for cout, cin, mb, nb, strip, wgs, w in [(288, 288, 1, 1, 128, 2 * cus, W),
+                                             (288, 864, 1, 1, 128, 2 * cus, W),
+                                             (576, 288, 2, 1, 128, cus, W // 2),
+                                             (576, 576, 2, 2, 64, cus, W // 2)]:
+        assert -(-w // strip) > wgs // (cout // (32 * mb) * (cin // (32 * nb)))
+    net, ref = _net_and_ref(seed=41, levels=levels, base=base)
+    x, u = _inputs(1, H, W, seed=42)
+    loss = net.loss_grad(torch.from_numpy(x).cuda(), torch.from_numpy(u).cuda())
+    g = net.grads()
+    Lr, gr = U.loss_and_grads(ref, _c2(x), _c2(u), levels)
+    assert abs(loss - Lr) / Lr < 1e-2
+    for k in gr:
+        a, b = g[k].astype(np.float64).ravel(), gr[k].ravel()
+        rel = np.linalg.norm(a - b) / np.linalg.norm(b)
+        say(f"   {k:8s} rel err {rel:.2e}")
+        assert rel < (0.2 if k.startswith("e0a") else 6e-2), k
+
+
+def test_gradients_repeat_bit_for_bit():
+    """Every gradient sum runs in a fixed order: the same inputs give the same
+    bits, also after a step on another shape (other buffers)."""
+    net, _ = _net_and_ref(seed=51, levels=3)
+    x, u = (torch.from_numpy(a).cuda() for a in _inputs(3, 48, 132, seed=52))
+    x2, u2 = (torch.from_numpy(a).cuda() for a in _inputs(1, 16, 260, seed=53))
+    first = (net.loss_grad(x, u), net.get_flat(grads=True))
+    net.loss_grad(x2, u2)
+    for _ in range(3):
+        loss = net.loss_grad(x, u)
+        assert loss == first[0] and np.array_equal(net.get_flat(grads=True), first[1])
+
+
+def test_seeded_weights_are_the_standard_normal_draws():
+    """A network made from a seed has He-normal weights drawn layer by layer
+    from the 64-bit Mersenne twister by the polar method, second coordinate
+    first (what std::normal_distribution<double> of libstdc++ draws), zero
+    biases and a zero output layer."""
+    M = (1 << 64) - 1
+
+    class Twister:
+        def __init__(self, seed):
+            self.s, self.i = [seed & M], 312
+            for k in range(1, 312):
+                p = self.s[-1]
+                self.s.append((6364136223846793005 * (p ^ (p >> 62)) + k) & M)
+
+        def __call__(self):
+            if self.i == 312:
+                s = self.s
+                for k in range(312):
+                    y = (s[k] & ~0x7FFFFFFF & M) | (s[(k + 1) % 312] & 0x7FFFFFFF)
+                    s[k] = s[(k + 156) % 312] ^ (y >> 1) ^ (0xB5026F5AA96619E9 if y & 1 else 0)
+                self.i = 0
+            y = self.s[self.i]
+            self.i += 1
+            y ^= (y >> 29) & 0x5555555555555555
+            y ^= (y << 17) & 0x71D67FFFEDA60000
+            y ^= (y << 37) & 0xFFF7EEE000000000
+            return y ^ (y >> 43)
+
+    for seed in (0, 12345678901234567890):
+        p = glsu.UNet(2, 32, seed=seed).params()
+        rng = Twister(seed)
+
+        def unit():
+            return 2.0 * min(float(rng()) / 2.0 ** 64, math.nextafter(1.0, 0.0)) - 1.0
+
+        for name, kind, ci, co in glsu.learned.layer_specs(2, 32):
+            assert not p[name + ".b"].any()
+            if name == "out":
+                assert not p[name + ".w"].any()
+                continue
+            sd, want = math.sqrt(2.0 / (9 * ci)), []
+            for _ in range(0, 9 * ci * co, 2):
+                while True:
+                    a, b = unit(), unit()
+                    r2 = a * a + b * b
+                    if 0.0 < r2 <= 1.0:
+                        break
+                m = math.sqrt(-2.0 * math.log(r2) / r2)
+                want += [b * m * sd, a * m * sd]
+            assert np.array_equal(p[name + ".w"].ravel(), np.float32(want)), (seed, name)
