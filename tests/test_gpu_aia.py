@@ -133,3 +133,67 @@ def test_many_iterations_poll_and_errors(oracle):
         glsu.AIA(2, W, H)
     with pytest.raises(ValueError):
         a(torch.from_numpy(f[:4]).cuda())
+
+
+@pytest.mark.parametrize("max_iter", [1, 2, 3, 4])
+def test_iteration_limits_around_the_launch_lead(oracle, max_iter):
+    """The host enqueues two iterations ahead of the completed ones: limits
+    below, at and above that lead stop at the oracle's iteration and shifts
+    (bars as above)."""
+    M, H, W = 6, 70, 58
+    f, _, _ = aia_frames(M, H, W, 41, noise=8.0, dtype=np.float32)
+    start = np.array([0, 0.8, 2.1, -1.1, 2.9, -2.0], np.float32)
+    p_ref, d_ref, it_ref, err_ref = oracle.aia(f.astype(np.float64), start.astype(np.float64),
+                                               max_iter, 1e-9)
+    a = glsu.AIA(M, W, H)
+    fr = torch.from_numpy(f).cuda()
+    for _ in range(2):
+        phi, d, _, it, err = a(fr, deltas=start, max_iter=max_iter, max_err=1e-9)
+        say(f"[aia limit {max_iter}] {it} it, err {err:.2e} (oracle {it_ref}, {err_ref:.2e})")
+        assert it == it_ref == max_iter
+        assert np.abs(wrap(d - d_ref)).max() < 2e-5
+        assert wrapped_err(phi.cpu().numpy(), p_ref)[0] < 1e-4
+
+
+def test_run_behind_long_work_on_the_stream():
+    """Work queued before the run keeps the first iteration from reporting for
+    longer than the host polls for it (2 ms), so it waits for the stream
+    instead; same bits as on an idle stream."""
+    M, H, W = 8, 200, 150
+    f, _, _ = aia_frames(M, H, W, 43, dtype=np.uint8)
+    fr = torch.from_numpy(f).cuda()
+    a = glsu.AIA(M, W, H)
+    phi, d, _, it, err = a(fr, seed=5)
+    assert it > 3
+    m = torch.ones((4096, 4096), device="cuda")
+    out = torch.empty_like(m)
+    torch.mm(m, m, out=out)
+    e0, e1 = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+    torch.cuda.synchronize()
+    e0.record()
+    for _ in range(60):  # 137 GFLOP each
+        torch.mm(m, m, out=out)
+    e1.record()
+    phi2, d2, _, it2, err2 = a(fr, seed=5)
+    busy = e0.elapsed_time(e1)
+    say(f"[aia busy] {busy:.1f} ms queued before; {it2} it")
+    assert busy > 10
+    assert torch.equal(phi, phi2) and np.array_equal(d, d2) and it == it2 and err == err2
+
+
+def test_singular_shift_step_is_reported_from_the_device():
+    """Black frames: every pixel has the same phase, so the first shift step's
+    matrix is singular (the initial shifts are distinct, so the phase step on
+    the host passes); the handle runs correctly afterwards."""
+    M, H, W = 5, 64, 96
+    f, _, _ = aia_frames(M, H, W, 47, dtype=np.uint8)
+    fr = torch.from_numpy(f).cuda()
+    start = np.array([0, 1.0, -1.0, 2.0, -2.5], np.float32)
+    a = glsu.AIA(M, W, H)
+    want = a(fr, deltas=start)
+    for _ in range(2):
+        with pytest.raises(glsu.NotPositiveDefiniteError, match="shift step"):
+            a(torch.zeros_like(fr), deltas=start)
+        got = a(fr, deltas=start)
+        assert torch.equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        assert got[3:] == want[3:]
