@@ -1117,11 +1117,6 @@ int live_fit(int plan, int n) {
     if (q.id == plan) return n <= live_regs(q.E) * q.T ? 1 : 0;
   return 0;
 }
-int plan_lanes(int plan) {
-  for (const FftPlanInfo& q : fft_plans())
-    if (q.id == plan) return q.T;
-  return 0;
-}
 
 // Default column plans of a batch.  One launch carries the columns of every
 // image of a class, so the rule of plan_default_cols takes the columns of them
@@ -1228,7 +1223,7 @@ extern "C" int glsu_dpra_batch_create(glsu_dpra_batch** out, const glsu_seq_desc
     for (const FftPlanInfo& q : fft_plans())
       if (q.id == keys[c].px) E = q.E;
     if (keys[c].rw < 0) keys[c].rw = rows_waves_default(E, rows);
-    if (keys[c].cw < 0) keys[c].cw = cols_waves_default(plan_lanes(keys[c].py), items);
+    if (keys[c].cw < 0) keys[c].cw = cols_waves_default(keys[c].py, items);
     std::string err;
     int rc = wff_plan_init(bc.p, seqs[first].width, seqs[first].height, pr->sigma_x, pr->wxl,
                            pr->wxh, pr->wxi, pr->sigma_y, pr->wyl, pr->wyh, pr->wyi, pr->thr,

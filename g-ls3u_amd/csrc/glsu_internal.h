@@ -92,9 +92,9 @@ int wff_plan_geometry(WffPlan& p, int W, int H, double sigx, double wxl, double 
                       int plany, int cols_waves, int rows_waves, const char** err);
 // Default column plan of the filter for `items` columns over all planes.
 int plan_default_cols(int need, double items);
-// Default waves per workgroup of the column kernel for `items` columns and a
-// plan of T lanes per transform.
-int cols_waves_default(int T, double items);
+// Default waves per workgroup of the column kernel for `items` columns on a
+// compiled plan.
+int cols_waves_default(int plan, double items);
 // Default waves per row of the row kernels for `rows` rows in one launch and a
 // plan of E points per lane.
 int rows_waves_default(int E, int rows);

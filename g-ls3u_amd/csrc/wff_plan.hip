@@ -342,14 +342,20 @@ int rows_waves_default(int E, int rows) {
 
 // Waves per workgroup of the column kernel.  Workgroups of four waves share one
 // twiddle table best; a launch of few wavefronts (columns / transforms per
-// wavefront) spreads more evenly over the CUs in pairs.  Measured, column
-// kernel, us, 2 / 4 waves a workgroup: 512 points, 1400 wavefronts 19.3 / 20.4,
-// 2150 24.4 / 25.6, 2600 27.5 / 26.8, 3200 30.4 / 31.6, 5200 (1024 x 1024, 1280
-// points) 127 / 121; four 320-point transforms a wavefront, 1300 35.8 / 40.1,
-// 1750 40.3 / 41.2.  Between 2050 and 3072 wavefronts it goes either way by 2 to
-// 5 % with the remainder of the last round; from 1024 points up four waves are
-// ahead there (2050 wavefronts 56.2 / 49.7, 2600 62.8 / 61.7).
-int cols_waves_default(int T, double items) { return items * T < 3072 * 64 ? 2 : 4; }
+// wavefront) spreads more evenly over the CUs in pairs, as long as the chains
+// are short: from 768 points up two pairs on a CU slow each other.  Measured,
+// column kernel, us, 2 / 4 waves a workgroup: 512 points, 1400 wavefronts 19.3 /
+// 20.4, 2150 24.4 / 25.6, 2600 27.5 / 26.8, 3200 30.4 / 31.6, 5200 (1024 x 1024,
+// 1280 points) 127 / 121; four 320-point transforms a wavefront, 1300 35.8 /
+// 40.1, 1750 40.3 / 41.2.  Whole filter: 200 x 900 (1000 wavefronts of 1024
+// points) 48.1 / 45.0, 200 x 1200 (1280 points) 60.8 / 54.9, 170 x 600 (768) 6 %;
+// above them to 3072 wavefronts 0 to 5 %, the other way by 1 to 3 % from 1050 to
+// 1550.  Up to 512 points pairs win below 2500 wavefronts (by 0 to 5 %) and lose
+// up to 3 % from there to the line.
+int cols_waves_default(int plan, double items) {
+  const PlanRow* p = plan_row(plan);
+  return p->N <= 512 && items * p->T < 3072 * 64 ? 2 : 4;
+}
 
 int wff_plan_geometry(WffPlan& p, int W, int H, double sigx, double wxl, double wxh, double wxi,
                       double sigy, double wyl, double wyh, double wyi, double thr, int planx,
@@ -392,7 +398,7 @@ int wff_plan_geometry(WffPlan& p, int W, int H, double sigx, double wxl, double 
   if (rows_waves < 1 || rows_waves > kRowWavesMax) rows_waves = rows_waves_default(px->E, H);
   p.rows_waves = std::min(rows_waves, p.nwx);
   if (cols_waves != 1 && cols_waves != 2 && cols_waves != 4)
-    cols_waves = cols_waves_default(py->T, (double)p.nwx * W);
+    cols_waves = cols_waves_default(plany, (double)p.nwx * W);
   p.cols_waves = cols_waves;
   // keep dynamic LDS per workgroup within 64 KiB
   while (p.cols_waves > 1 && plan_smem_bytes(plany, p.cols_waves, true) > 65536) p.cols_waves /= 2;

@@ -193,3 +193,26 @@ def test_default_column_plan_of_short_images_matches_oracle(oracle, W, H, N):
     say(f"   {W}x{H} {w.tuning()} rel={rel:.2e} phase rms={rms:.2e}")
     assert rel < 1e-4
     assert rms < 1e-4
+
+
+@pytest.mark.parametrize("W,H,waves", [
+    (200, 480, 2),    # 512 points, 1000 wavefronts: pairs
+    (200, 483, 4),    # one row more: 768 points
+    (200, 1000, 4),   # 1280 points
+    (614, 482, 2),    # 3070 wavefronts
+    (615, 482, 4),    # 3075
+])
+def test_default_column_workgroups_at_their_limits(W, H, waves):
+    """Waves per workgroup of the column kernel by the plan's length and the
+    wavefronts of the launch; the shape must not change the result."""
+    rng = np.random.default_rng(W)
+    f = np.exp(1j * rng.normal(0, 0.8, (H, W))).astype(np.complex64)
+    params = glsu.wff_params(10.0, -0.2, 0.2, 0.1)
+    w = glsu.WFT2(W, H, params=params)
+    t = w.tuning()
+    say(f"   {W}x{H} {t}")
+    assert t["cols_waves"] == waves
+    x = torch.from_numpy(f).cuda()
+    o = glsu.WFT2(W, H, params=params, tuning=dict(t, cols_waves=6 - waves))
+    assert o.tuning()["cols_waves"] == 6 - waves
+    assert torch.equal(w(x), o(x))
